@@ -203,12 +203,18 @@ __global__ void factor_prep_kernel(const float* __restrict__ f, int K, float* __
   rcp[k] = 1.0f / v;
 }
 
-bool fast_path_ok(const ic_rotq_args& a) {
+// Forms the fast path takes: 16-bit rows of whole 16-value runs, 16-byte
+// aligned, without the old-SmoothQuant divide, quantized or (quant false)
+// written in the activation type.  Measured at 4608 x 3072, R = 256 with
+// factors and perm, f16, not quantized: rotate_quant_kernel 61.9 us, the fast
+// kernel 27.9 us (quantized, the two were apart before already).
+bool fast_path_ok(const ic_rotq_args& a, bool quant = true) {
   auto al16 = [](const void* p) { return (((uintptr_t)p) & 15) == 0; };
   if (a.dtype != IC_DTYPE_F16 && a.dtype != IC_DTYPE_BF16) return false;
-  if (a.sm_rcp != nullptr || a.q_out == nullptr) return false;
+  if (a.sm_rcp != nullptr || (quant ? a.q_out : a.y_out) == nullptr) return false;
   if (a.K_in % 16 || a.K_w % 16 || a.K_w > (int64_t)kFastMaxTiles * kTile) return false;
-  if (a.ldx % 8 || a.ldq % 16 || !al16(a.x) || !al16(a.q_out)) return false;
+  if (a.ldx % 8 || !al16(a.x)) return false;
+  if (quant ? (a.ldq % 16 || !al16(a.q_out)) : (a.ldy % 8 || !al16(a.y_out))) return false;
   if ((a.sr_rcp && !al16(a.sr_rcp)) || (a.perm && !al16(a.perm))) return false;
   return true;
 }
@@ -300,6 +306,11 @@ static int run_rotq(const ic_rotq_args* a, bool quant, void* stream) {
   hipError_t e = hipErrorInvalidValue;
   if (quant && fast_path_ok(*a)) {
     e = a->dtype == IC_DTYPE_F16 ? ic_rq_fast_f16(*a, st) : ic_rq_fast_bf16(*a, st);
+    if (e != hipSuccess) return ic_set_error(IC_ERR_LAUNCH, "%s: %s", who, hipGetErrorString(e));
+    return IC_OK;
+  }
+  if (!quant && fast_path_ok(*a, false)) {
+    e = a->dtype == IC_DTYPE_F16 ? ic_rq_prep_f16(*a, st) : ic_rq_prep_bf16(*a, st);
     if (e != hipSuccess) return ic_set_error(IC_ERR_LAUNCH, "%s: %s", who, hipGetErrorString(e));
     return IC_OK;
   }

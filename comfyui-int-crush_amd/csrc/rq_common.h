@@ -291,6 +291,11 @@ hipError_t ic_rq_fast_bf16_plain(const ic_rotq_args& a, hipStream_t st);
 // with both SmoothRot factors and perm
 hipError_t ic_rq_fast_f16_both(const ic_rotq_args& a, hipStream_t st);
 hipError_t ic_rq_fast_bf16_both(const ic_rotq_args& a, hipStream_t st);
+// without quantization: the prepared row in the activation type (y_out)
+hipError_t ic_rq_prep_f16(const ic_rotq_args& a, hipStream_t st);
+hipError_t ic_rq_prep_bf16(const ic_rotq_args& a, hipStream_t st);
+hipError_t ic_rq_prep_f16_both(const ic_rotq_args& a, hipStream_t st);
+hipError_t ic_rq_prep_bf16_both(const ic_rotq_args& a, hipStream_t st);
 // with the row normalisation of a.norm first (rq_norm_{f16,bf16}.hip)
 hipError_t ic_rq_norm_f16(const ic_rotq_args& a, hipStream_t st);
 hipError_t ic_rq_norm_bf16(const ic_rotq_args& a, hipStream_t st);

@@ -105,12 +105,20 @@ constexpr int rq_fast_min_wgs() {
   if (TH >= 768 || (TH >= 448 && NT >= 2 && !wave_local)) return 1;
   return (NT <= 3 || VAR == kRqPlain) ? 2 : 1;
 }
-template <int DT, int LOG4R, int NT, int VAR, int TH, int NORM = 0>
+//
+// QUANT false (ic_prepare_activation): the prepared row itself leaves, in DT,
+// gathered from the same row buffer; no abs-max and no codes.  One workgroup
+// per row and a re-read of factors and perm for each row (rotate_quant_kernel,
+// which still serves the forms this kernel does not take) took 61.9 us for
+// 4608 x 3072 at R = 256 with both, this kernel 27.9 us.
+template <int DT, int LOG4R, int NT, int VAR, int TH, int NORM = 0, bool QUANT = true>
 __global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) void rq_fast_kernel(
     const u16* __restrict__ x, int64_t ldx, int M, int K_in, int K_r,
     const float* __restrict__ sr_rcp, const float* __restrict__ sr_f, int K_w,
     const int32_t* __restrict__ perm, int8_t* __restrict__ q_out, int64_t ldq,
-    float* __restrict__ s_out, const float* __restrict__ nw, const float* __restrict__ nb, float eps) {
+    float* __restrict__ s_out, const float* __restrict__ nw, const float* __restrict__ nb, float eps,
+    u16* __restrict__ y_out, int64_t ldy) {
+  static_assert(QUANT || NORM == 0, "the normalising kernels quantize");
   constexpr int RC = LOG4R <= 2 ? 0 : (LOG4R <= 4 ? 1 : (LOG4R == 5 ? 3 : 2));
   constexpr bool XCH = LOG4R >= 3;
   constexpr int kTile = TH * 16;  // positions per tile
@@ -253,9 +261,10 @@ __global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) vo
   auto wlr_off = [](int c, int q) { return 4096 + 2176 * c + 2 * (q + 16 * (q >> 8)); };
   static_assert(!WLR || 4096 + 2176 * NT <= 8 * 1216, "WLR rows fit the exchange slice");
   // Vector-memory operations each wave issues after its DMA of a row: one
-  // 16-byte code store per tile that every lane of every wave stores (plus,
-  // on some waves, pad-tile stores and the scale store, which only add).
-  const int kStoresAfterDma = min(K_w / kTile, NT);
+  // 16-byte code store (two without quantization) per tile that every lane of
+  // every wave stores (plus, on some waves, pad-tile stores and the scale
+  // store, which only add).
+  const int kStoresAfterDma = min(K_w / kTile, NT) * (QUANT ? 1 : 2);
   if constexpr (!PLAIN) {
     if constexpr (kDma) {
       // the constants' loads complete here (the compiler waits for them
@@ -429,7 +438,13 @@ __global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) vo
                 unpack8<DT>(xb, xo + 8);
               }
 #pragma unroll
-              for (int j = 0; j < 16; ++j) xs[j] = div_round_dt<DT>(xo[j], rc[PLAIN ? 0 : c][j], sr_f, p0 + j);
+              for (int j = 0; j < 16; ++j) {
+                xs[j] = div_round_dt<DT>(xo[j], rc[PLAIN ? 0 : c][j], sr_f, p0 + j);
+                // unrotated rows that leave unquantized keep the quotient's sign
+                // on a zero (the mixed-precision FMA that forms x * rcp adds +0)
+                if (!QUANT && LOG4R == 0 && xs[j] == 0.0f)
+                  xs[j] = __uint_as_float((__float_as_uint(xo[j]) ^ __float_as_uint(rc[PLAIN ? 0 : c][j])) & 0x80000000u);
+              }
             } else {
 #pragma unroll
               for (int j = 0; j < 16; ++j) xs[j] = 0.0f;
@@ -605,43 +620,77 @@ __global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) vo
     if constexpr (kDma) {
       if (next < M) stage_row(next);  // every exchange read of this row has returned
     }
-    // ---- row scale: RN_dt is monotone, so max |RN_dt(z)| = RN_dt(max |z|)
-    amax = wave_max_nonneg(amax);
-    if ((t & 63) == 0) red[t >> 6] = amax;
-    __syncthreads();
-    float mr = red[0];
+    float s = 1.0f, rcp_s = 1.0f;
+    if constexpr (QUANT) {
+      // ---- row scale: RN_dt is monotone, so max |RN_dt(z)| = RN_dt(max |z|)
+      amax = wave_max_nonneg(amax);
+      if ((t & 63) == 0) red[t >> 6] = amax;
+      __syncthreads();
+      float mr = red[0];
 #pragma unroll
-    for (int w = 1; w < TH / 64; ++w) mr = __builtin_fmaxf(mr, red[w]);
-    const float m = round_to_dt<DT>(mr);
-    const float s = quant_scale(m);
-    const float rcp_s = 1.0f / s;
-    if (t == 0) s_out[row] = s;
+      for (int w = 1; w < TH / 64; ++w) mr = __builtin_fmaxf(mr, red[w]);
+      const float m = round_to_dt<DT>(mr);
+      s = quant_scale(m);
+      rcp_s = 1.0f / s;
+      if (t == 0) s_out[row] = s;
+    } else if constexpr (WLR) {
+      // each wave reads back only what it wrote
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+      __syncthreads();
+    }
 
-    // ---- gather + quantize + store 16 codes per run
+    // ---- gather + quantize + store 16 codes (or 16 values) per run
     int8_t* qrow = q_out + (int64_t)row * ldq;
 #pragma unroll
     for (int c = 0; c < NT; ++c) {
       if (c * kTile >= K_w) break;  // uniform
       const int o0 = 16 * (t + TH * c);
-      float vv[16];
+      u16 g[16];  // gathered bits (has_perm)
+      v4u ra{}, rb{};
       if (has_perm) {
-        const char* rb = (const char*)rowbuf;
+        const char* src = (const char*)rowbuf;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          vv[2 * i] = bits16_f32<DT>(*(const u16*)(rb + (po[PLAIN ? 0 : c][i] & 0xffffu)));
-          vv[2 * i + 1] = bits16_f32<DT>(*(const u16*)(rb + (po[PLAIN ? 0 : c][i] >> 16)));
+          g[2 * i] = *(const u16*)(src + (po[PLAIN ? 0 : c][i] & 0xffffu));
+          g[2 * i + 1] = *(const u16*)(src + (po[PLAIN ? 0 : c][i] >> 16));
         }
       } else if constexpr (WLR) {
         // this lane's 16 consecutive positions are wave-local 16 lane .. 16 lane + 15
         const char* wl = slice + wlr_off(c, 16 * lane);
-        unpack8<DT>(*(const v4u*)wl, vv);
-        unpack8<DT>(*(const v4u*)(wl + 16), vv + 8);
+        ra = *(const v4u*)wl;
+        rb = *(const v4u*)(wl + 16);
       } else {
-        unpack8<DT>(*(const v4u*)(rowbuf + rbaddr(o0)), vv);
-        unpack8<DT>(*(const v4u*)(rowbuf + rbaddr(o0) + 8), vv + 8);
+        ra = *(const v4u*)(rowbuf + rbaddr(o0));
+        rb = *(const v4u*)(rowbuf + rbaddr(o0) + 8);
       }
-      const v4u codes = quant16(vv, s, rcp_s);
-      if (o0 < K_w) *(v4u*)(qrow + o0) = codes;
+      if constexpr (QUANT) {
+        float vv[16];
+        if (has_perm) {
+#pragma unroll
+          for (int j = 0; j < 16; ++j) vv[j] = bits16_f32<DT>(g[j]);
+        } else {
+          unpack8<DT>(ra, vv);
+          unpack8<DT>(rb, vv + 8);
+        }
+        const v4u codes = quant16(vv, s, rcp_s);
+        if (o0 < K_w) *(v4u*)(qrow + o0) = codes;
+      } else {
+        if (has_perm) {
+          uint32_t w[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) w[i] = (uint32_t)g[2 * i] | ((uint32_t)g[2 * i + 1] << 16);
+          ra = v4u{w[0], w[1], w[2], w[3]};
+          rb = v4u{w[4], w[5], w[6], w[7]};
+        }
+        if (o0 < K_w) {
+          v4u* dst = (v4u*)(y_out + (int64_t)row * ldy + o0);
+          dst[0] = ra;
+          dst[1] = rb;
+        }
+      }
       __builtin_amdgcn_sched_barrier(0);  // one run at a time keeps the register footprint small
     }
   }
@@ -744,50 +793,50 @@ int persistent_grid(int threads, int64_t M) {
   return (int)(M < g ? M : g);
 }
 
-template <int DT, int LOG4R, int NT, int VAR, int TH = kThreads, int NORM = 0>
+template <int DT, int LOG4R, int NT, int VAR, int TH = kThreads, int NORM = 0, bool QUANT = true>
 hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
-  constexpr auto kern = rq_fast_kernel<DT, LOG4R, NT, VAR, TH, NORM>;
+  constexpr auto kern = rq_fast_kernel<DT, LOG4R, NT, VAR, TH, NORM, QUANT>;
   const int64_t K_r = LOG4R == 0 ? a.K_in : ((a.K_in + a.rot_size - 1) / a.rot_size) * a.rot_size;
   kern<<<dim3(persistent_grid<kern>(TH, a.M)), dim3(TH), 0, st>>>(
       (const u16*)a.x, a.ldx, (int)a.M, (int)a.K_in, (int)K_r, a.sr_rcp, a.sr_f, (int)a.K_w, a.perm,
-      a.q_out, a.ldq, a.s_out, a.nw, a.nb, a.eps);
+      a.q_out, a.ldq, a.s_out, a.nw, a.nb, a.eps, (u16*)a.y_out, a.ldy);
   return hipGetLastError();
 }
 
-template <int DT, int LOG4R, int VAR, int NORM = 0>
+template <int DT, int LOG4R, int VAR, int NORM = 0, bool QUANT = true>
 hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
   if constexpr (LOG4R == 5) {
     // five one-block waves cover 4097..5120 values in one tile (Wan's 5120
     // would otherwise take two 4096-tiles, 37.5 % of them padding)
-    if (a.K_w > kTile && a.K_w <= 320 * 16) return launch_fast_t<DT, LOG4R, 1, VAR, 320, NORM>(a, st);
+    if (a.K_w > kTile && a.K_w <= 320 * 16) return launch_fast_t<DT, LOG4R, 1, VAR, 320, NORM, QUANT>(a, st);
     // seven one-block waves, two tiles: 12289..14336 values (Wan's FFN-down
     // 14336 instead of four 4096-tiles; ~99 KB of LDS, one workgroup per CU)
-    if (a.K_w > 3 * kTile && a.K_w <= 2 * 448 * 16) return launch_fast_t<DT, LOG4R, 2, VAR, 448, NORM>(a, st);
+    if (a.K_w > 3 * kTile && a.K_w <= 2 * 448 * 16) return launch_fast_t<DT, LOG4R, 2, VAR, 448, NORM, QUANT>(a, st);
   }
   if constexpr (LOG4R >= 3 && LOG4R <= 5) {
     // one tile of twelve waves for 8193..12288 values (Flux's 12288): the
     // per-thread constants of one tile instead of three
-    if (a.K_w > 2 * kTile && a.K_w <= 768 * 16) return launch_fast_t<DT, LOG4R, 1, VAR, 768, NORM>(a, st);
+    if (a.K_w > 2 * kTile && a.K_w <= 768 * 16) return launch_fast_t<DT, LOG4R, 1, VAR, 768, NORM, QUANT>(a, st);
     // two tiles of eight waves for 12289..16384 (Flux's single-block 15360)
-    if (a.K_w > 3 * kTile) return launch_fast_t<DT, LOG4R, 2, VAR, 512, NORM>(a, st);
+    if (a.K_w > 3 * kTile) return launch_fast_t<DT, LOG4R, 2, VAR, 512, NORM, QUANT>(a, st);
   }
   if constexpr (LOG4R <= 5) {
     // three-wave workgroups where their tile fits the row more tightly
     // (3072: one full tile instead of 3/4 of one; 4097..6144: two)
     constexpr int T3 = 192 * 16;
-    if (a.K_w <= T3 && a.K_w > kTile / 2) return launch_fast_t<DT, LOG4R, 1, VAR, 192, NORM>(a, st);
-    if (a.K_w > kTile && a.K_w <= 2 * T3) return launch_fast_t<DT, LOG4R, 2, VAR, 192, NORM>(a, st);
+    if (a.K_w <= T3 && a.K_w > kTile / 2) return launch_fast_t<DT, LOG4R, 1, VAR, 192, NORM, QUANT>(a, st);
+    if (a.K_w > kTile && a.K_w <= 2 * T3) return launch_fast_t<DT, LOG4R, 2, VAR, 192, NORM, QUANT>(a, st);
   }
-  if (a.K_w <= kTile) return launch_fast_t<DT, LOG4R, 1, VAR, kThreads, NORM>(a, st);
-  if (a.K_w <= 2 * kTile) return launch_fast_t<DT, LOG4R, 2, VAR, kThreads, NORM>(a, st);
-  if (a.K_w <= 3 * kTile) return launch_fast_t<DT, LOG4R, 3, VAR, kThreads, NORM>(a, st);
-  return launch_fast_t<DT, LOG4R, 4, VAR, kThreads, NORM>(a, st);
+  if (a.K_w <= kTile) return launch_fast_t<DT, LOG4R, 1, VAR, kThreads, NORM, QUANT>(a, st);
+  if (a.K_w <= 2 * kTile) return launch_fast_t<DT, LOG4R, 2, VAR, kThreads, NORM, QUANT>(a, st);
+  if (a.K_w <= 3 * kTile) return launch_fast_t<DT, LOG4R, 3, VAR, kThreads, NORM, QUANT>(a, st);
+  return launch_fast_t<DT, LOG4R, 4, VAR, kThreads, NORM, QUANT>(a, st);
 }
 
 // VAR must match the arguments (the per-dtype dispatcher routes on them).
-template <int DT, int VAR, int NORM = 0>
+template <int DT, int VAR, int NORM = 0, bool QUANT = true>
 hipError_t launch_fast(const ic_rotq_args& a, hipStream_t st) {
-  if (NORM == 0 && VAR == kRqPlain && a.rot_size == 0 && a.K_w == a.K_in && a.K_in <= 32 * 512) {
+  if (QUANT && NORM == 0 && VAR == kRqPlain && a.rot_size == 0 && a.K_w == a.K_in && a.K_in <= 32 * 512) {
     const unsigned grid = (unsigned)((a.M + 3) / 4);
     if (a.K_in <= 8 * 512)
       quant_wave_kernel<DT, 8><<<grid, kThreads, 0, st>>>((const u16*)a.x, a.ldx, (int)a.M, (int)a.K_in, a.q_out, a.ldq, a.s_out);
@@ -798,12 +847,12 @@ hipError_t launch_fast(const ic_rotq_args& a, hipStream_t st) {
     return hipGetLastError();
   }
   switch (a.rot_size) {
-    case 0: return launch_fast_nt<DT, 0, VAR, NORM>(a, st);
-    case 16: return launch_fast_nt<DT, 2, VAR, NORM>(a, st);
-    case 64: return launch_fast_nt<DT, 3, VAR, NORM>(a, st);
-    case 256: return launch_fast_nt<DT, 4, VAR, NORM>(a, st);
-    case 1024: return launch_fast_nt<DT, 5, VAR, NORM>(a, st);
-    case 4096: return launch_fast_nt<DT, 6, VAR, NORM>(a, st);
+    case 0: return launch_fast_nt<DT, 0, VAR, NORM, QUANT>(a, st);
+    case 16: return launch_fast_nt<DT, 2, VAR, NORM, QUANT>(a, st);
+    case 64: return launch_fast_nt<DT, 3, VAR, NORM, QUANT>(a, st);
+    case 256: return launch_fast_nt<DT, 4, VAR, NORM, QUANT>(a, st);
+    case 1024: return launch_fast_nt<DT, 5, VAR, NORM, QUANT>(a, st);
+    case 4096: return launch_fast_nt<DT, 6, VAR, NORM, QUANT>(a, st);
   }
   return hipErrorInvalidValue;
 }
