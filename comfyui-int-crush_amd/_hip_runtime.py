@@ -89,6 +89,9 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "ic_gemm_w4a16": ([_P, _I, _L, _L, _L, _P, _L, _L, _P, _L, _P, _I, _P, _L, _P], _I),
     "ic_w4a16_stage_layout": ([_P, _L, _L, _L, _P, _L, _P, _P, _P], _I),
     "ic_gemm_w4a16_staged": ([_P, _I, _L, _L, _L, _P, _L, _P, _L, _P, _I, _P, _L, _P], _I),
+    "ic_gemm_w4a16_splitk_bytes": ([_L, _L, _L, _L], _L),
+    "ic_gemm_w4a16_ws": ([_P, _I, _L, _L, _L, _P, _L, _L, _P, _L, _P, _I, _P, _L, _P, _L, _P], _I),
+    "ic_gemm_w4a16_staged_ws": ([_P, _I, _L, _L, _L, _P, _L, _P, _L, _P, _I, _P, _L, _P, _L, _P], _I),
     "ic_unpack_int4_to_int8": ([_P, _L, _L, _L, _P, _L, _P], _I),
     "ic_unpack_int4_to_float": ([_P, _P, _L, _L, _L, _L, _P, _I, _L, _P], _I),
     "ic_f6_activation_bytes": ([_L, _L], _L),
@@ -527,6 +530,14 @@ def _splitk_workspace(M: int, N: int, K: int, G: int, int4: bool, device) -> tup
     return torch.empty(nb, dtype=torch.uint8, device=device), nb
 
 
+def _w16_workspace(M: int, N: int, K: int, G: int, device) -> tuple[torch.Tensor | None, int]:
+    """The same for the W4A16 GEMM (ic_gemm_w4a16_splitk_bytes)."""
+    nb = int(lib().ic_gemm_w4a16_splitk_bytes(M, N, K, G))
+    if nb <= 0:
+        return None, 0
+    return torch.empty(nb, dtype=torch.uint8, device=device), nb
+
+
 # Epilogue activation codes (kernels/triton_int8_gemm.py:24-27 for 0-2).
 ACT_NONE, ACT_SILU, ACT_GELU, ACT_GELU_TANH = 0, 1, 2, 3
 
@@ -890,8 +901,9 @@ def gemm_w4a16(x: torch.Tensor, w_packed: torch.Tensor, s_w: torch.Tensor,
     bp, bdt, _keep = _bias_args(bias, N)
     c = _out_buffer(out, M, N, x2.dtype, x2.device)
     with torch.cuda.device(x2.device):
-        _call("ic_gemm_w4a16", _ptr(x2), dt, M, K, x2.stride(0), _ptr(w), N, w.stride(0), _ptr(sw), G,
-              bp, bdt, _ptr(c), c.stride(0), _stream(x2))
+        ws, nb = _w16_workspace(M, N, K, G, x2.device)
+        _call("ic_gemm_w4a16_ws", _ptr(x2), dt, M, K, x2.stride(0), _ptr(w), N, w.stride(0), _ptr(sw), G,
+              bp, bdt, _ptr(c), c.stride(0), _ptr(ws), nb, _stream(x2))
     return c
 
 
@@ -945,8 +957,9 @@ def gemm_w4a16_staged(x: torch.Tensor, w_staged: torch.Tensor, s_staged: torch.T
     bp, bdt, _keep = _bias_args(bias, N)
     c = _out_buffer(out, M, N, x2.dtype, x2.device)
     with torch.cuda.device(x2.device):
-        _call("ic_gemm_w4a16_staged", _ptr(x2), dt, M, K, x2.stride(0), _ptr(w_staged.contiguous()), N, _ptr(ss), G,
-              bp, bdt, _ptr(c), c.stride(0), _stream(x2))
+        ws, nb = _w16_workspace(M, N, K, G, x2.device)
+        _call("ic_gemm_w4a16_staged_ws", _ptr(x2), dt, M, K, x2.stride(0), _ptr(w_staged.contiguous()), N, _ptr(ss),
+              G, bp, bdt, _ptr(c), c.stride(0), _ptr(ws), nb, _stream(x2))
     return c
 
 

@@ -4,6 +4,18 @@
 #pragma once
 #include "ic_common.h"
 
+namespace ic_gemm {
+struct GemmArgs {
+  const int8_t* A; int64_t lda; const uint8_t* B; int64_t ldb;
+  const float* s_a; const float* s_w; int G;
+  const void* bias; int bias_dt; void* C; int out_dt; int64_t ldc; int M, N, K;
+  int32_t* acc_out; bool int4;
+  void* ws = nullptr; int64_t ws_bytes = 0;  // split-K workspace (optional)
+  ic_epi epi{};                              // activation / residual epilogue
+  bool kil = false;                          // packed INT4 in the K-interleaved nibble order
+};
+}  // namespace ic_gemm
+
 namespace {
 
 constexpr int kNT = 512;  // threads per workgroup

@@ -36,19 +36,8 @@
 
 #include "gemm_common.h"
 #include "gemm_i8_big.h"
+#include "gemm_mid_plan.h"
 #include "rq_common.h"
-
-namespace ic_gemm {
-struct GemmArgs {
-  const int8_t* A; int64_t lda; const uint8_t* B; int64_t ldb;
-  const float* s_a; const float* s_w; int G;
-  const void* bias; int bias_dt; void* C; int out_dt; int64_t ldc; int M, N, K;
-  int32_t* acc_out; bool int4;
-  void* ws = nullptr; int64_t ws_bytes = 0;  // split-K workspace (optional)
-  ic_epi epi{};                              // activation / residual epilogue
-  bool kil = false;                          // packed INT4 in the K-interleaved nibble order
-};
-}  // namespace ic_gemm
 
 // GEMM launches with the activation / residual epilogue compiled in
 // (gemm_i8_epi.hip).
@@ -912,9 +901,65 @@ hipError_t launch_big(const GemmArgs& g, hipStream_t st) {
   }
 }
 
+// Estimated microseconds of the launch the rules above choose (model and
+// constants as in gemm_mid_plan.h): rounds of workgroups x stages x the
+// stage time of a tile, 256 x 192 for the big kernel and scaled with its area.
+double big_us(int mode, int tmb, int64_t M, int64_t N, int KT) {
+  constexpr double stage[6] = {1.5, 1.8, 1.1, 1.1, 3.5, 1.6};  // by weight mode G128 ... G128I8
+  const int64_t cus = ic_num_cus();
+  const int64_t tiles = ((M + 32 * tmb - 1) / (32 * tmb)) * ((N + big::BN - 1) / big::BN);
+  return (double)((tiles + cus - 1) / cus) * (KT * stage[mode] * tmb / 8.0 + 4.0) + 5.0;
+}
+double tile_us(const GemmArgs& g, bool grouped, const TileShape& t, int S) {
+  const int64_t cus = ic_num_cus(), area = (int64_t)t.bm * t.bn / 16384;  // of 128 x 128
+  const int64_t n = (int64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn) * S;
+  // one 128 x 128 stage, and each further 128 x 128 of a larger tile
+  const double one = g.int4 ? (grouped ? 0.85 : 0.70) : (grouped ? 0.60 : 0.55);
+  const double more = g.int4 ? (grouped ? 0.30 : 0.25) : (grouped ? 0.45 : 0.35);
+  const int KT = g.K / kBK;
+  return kMidFixed + 1.0 + (double)((n + cus - 1) / cus) * ((KT + S - 1) / S) * (one + more * (area - 1)) +
+         (S > 1 ? kMidReduce + (double)S * g.M * g.N * 8.0 / kMidBytesPerUs : 0.0);
+}
+
+// The small tiles instead, where their estimate is below `base` (that of the
+// launch chosen otherwise, in S0 slices).  Grouped launches keep its slices:
+// a slice boundary moves the order of the fp32 fold, and the outputs of a
+// shape do not depend on the kernel (nor on the output type, whose f32 form
+// only the other tiles write).  Per-row sums are exact in any slices.
+bool mid_pick(const GemmArgs& g, int mode, bool grouped, int S0, double base, MidPlan& p) {
+  if (!mid_rounds_ok(g.M, g.N)) return false;
+  const int64_t mn4 = (int64_t)g.M * g.N * 4;
+  const int64_t fit = g.ws != nullptr ? g.ws_bytes / mn4 : 0;
+  const int most = fit > 16 ? 16 : (fit < 1 ? 1 : (int)fit);
+  p = grouped ? mid_plan(mode, g.M, g.N, g.K / kBK, S0, S0) : mid_plan(mode, g.M, g.N, g.K / kBK, 1, most);
+  return p.us < base;
+}
+// Groups of 64 or 32 columns, against the big tile; never split.
+bool mid_pick_unsplit(const GemmArgs& g, int mode, MidPlan& p) {
+  if (!mid_rounds_ok(g.M, g.N)) return false;
+  p = mid_plan(mode, g.M, g.N, g.K / kBK, 1, 1);
+  return p.us < big_us(mode, big_rows(g), g.M, g.N, g.K / kBK);
+}
+hipError_t launch_mid_any(const GemmArgs& g, int mode, const MidPlan& p, hipStream_t st) {
+  if (!g.int4) return ic_launch_mid_i8(g, mode, p.tile, p.S, st);
+  return g.kil ? ic_launch_mid_kil(g, mode, p.tile, p.S, st) : ic_launch_mid_i4(g, mode, p.tile, p.S, st);
+}
+
 template <bool INT4, int GS, int OUT_DT, bool ACC, bool EPI>
 hipError_t pick_tile(const GemmArgs& g, hipStream_t st) {
   const TileShape t = tile_choice(g, GS != 0);
+  if constexpr (!ACC && OUT_DT != IC_DTYPE_F32) {
+    if (g.C != nullptr && big_out_ok(g)) {
+      constexpr int mode = GS != 0 ? (INT4 ? big::G128 : big::G128I8) : (INT4 ? big::ROW4 : big::ROW8);
+      const bool use_big = GS != 0 ? big_tile_ok(g) : big_row_ok(g);
+      // as launch_mfma splits it
+      int S = g.ws != nullptr && !use_big ? splitk_plan(g, GS != 0) : 1;
+      if (g.ws_bytes < (int64_t)S * g.M * g.N * 4) S = 1;
+      MidPlan p;
+      if (mid_pick(g, mode, GS != 0, S, use_big ? big_us(mode, big_rows(g), g.M, g.N, g.K / kBK) : tile_us(g, GS != 0, t, S), p))
+        return launch_mid_any(g, mode, p, st);
+    }
+  }
   if constexpr (GS != 0 && !ACC && OUT_DT != IC_DTYPE_F32) {
     // grouped packed INT4, or grouped int8 weights (INT4 unpacked to bytes)
     if (big_tile_ok(g)) return launch_big<OUT_DT, EPI, INT4 ? big::G128 : big::G128I8>(g, st);
@@ -1054,13 +1099,17 @@ int run_gemm_t(GemmArgs g, hipStream_t st, const char* who, bool force_generic) 
   hipError_t e;
   if (!force_generic && big64_ok(g, gsize)) {
     // groups of 64 (or an odd multiple of 64) columns: the 288 x 192 kernel
-    // folding each 64-K step, at any M
-    if (g.out_dt == IC_DTYPE_F16) e = launch_big<IC_DTYPE_F16, EPI, big::G64>(g, st);
+    // folding each 64-K step, or the small tiles, at any M
+    MidPlan p;
+    if (mid_pick_unsplit(g, big::G64, p)) e = launch_mid_any(g, big::G64, p, st);
+    else if (g.out_dt == IC_DTYPE_F16) e = launch_big<IC_DTYPE_F16, EPI, big::G64>(g, st);
     else e = launch_big<IC_DTYPE_BF16, EPI, big::G64>(g, st);
   } else if (!force_generic && big32_ok(g, gsize)) {
     // groups of 32 (or an odd multiple of 32) columns: the same kernel folding
     // each 32-column half step
-    if (g.out_dt == IC_DTYPE_F16) e = launch_big<IC_DTYPE_F16, EPI, big::G32>(g, st);
+    MidPlan p;
+    if (mid_pick_unsplit(g, big::G32, p)) e = launch_mid_any(g, big::G32, p, st);
+    else if (g.out_dt == IC_DTYPE_F16) e = launch_big<IC_DTYPE_F16, EPI, big::G32>(g, st);
     else e = launch_big<IC_DTYPE_BF16, EPI, big::G32>(g, st);
   } else if (!force_generic && mfma_shape_ok(g, gsize)) {
     if constexpr (EPI) {

@@ -29,6 +29,7 @@
 #include "dequant4.h"
 #include "gemm_common.h"
 #include "gemm_i8_big.h"
+#include "gemm_mid_plan.h"
 
 namespace {
 
@@ -372,9 +373,48 @@ hipError_t launch_w4a16_big(const u16* A, int64_t lda, const uint8_t* B, int64_t
 }
 
 template <int DT>
+hipError_t launch_w16_mid(const u16* A, int64_t lda, const uint8_t* B, int64_t ldb, const float* s_w, int G,
+                          const void* bias, int bias_dt, u16* C, int64_t ldc, int M, int N, int K, void* ws,
+                          bool staged, const MidPlan& p, hipStream_t st) {
+  ic_gemm::GemmArgs g{(const int8_t*)A, lda * 2, B, ldb, nullptr, s_w, G, bias, bias_dt, C, DT, ldc, M, N, K,
+                      nullptr, true, ws, 0, ic_epi{}, staged};
+  return ic_launch_mid_w16(g, p.tile, p.S, st);
+}
+
+// Small tiles (gemm_mid.h) instead of the 256-row ones, or of the 128 x 256
+// tile for M <= 128, by the estimates of gemm_mid_plan.h: a 256 x 192 tile's
+// 64-K stage takes ~1.2 us, the 128 x 256 tile's ~1.15.
+MidPlan w16_plan(int64_t M, int64_t N, int64_t K, int max_s) {
+  MidPlan p = mid_plan(big::W16, M, N, (int)(K / 64), 1, max_s);
+  const int64_t cus = ic_num_cus();
+  double base = 1e30;
+  if (M > 128) {
+    for (int tmb = 8; tmb <= 10; ++tmb) {
+      const int64_t tiles = ((M + 32 * tmb - 1) / (32 * tmb)) * ((N + big::BN - 1) / big::BN);
+      const double us = (double)((tiles + cus - 1) / cus) * ((double)(K / 64) * 1.2 * tmb / 8.0 + 4.0) + 5.0;
+      if (us < base) base = us;
+    }
+  } else {
+    const int64_t tiles = (N + 255) / 256;
+    base = (double)((tiles + cus - 1) / cus) * (double)(K / 64) * 1.15 + 4.0;
+  }
+  if (base <= p.us || !mid_rounds_ok(M, N)) p.S = 0;  // the other tiles
+  return p;
+}
+constexpr int kW16MaxSplits = 16;
+int w16_max_splits(int64_t M, int64_t N, const void* ws, int64_t ws_bytes) {
+  const int64_t fit = ws != nullptr ? ws_bytes / (M * N * 4) : 0;
+  return fit > kW16MaxSplits ? kW16MaxSplits : (fit < 1 ? 1 : (int)fit);
+}
+
+template <int DT>
 hipError_t run_w4a16(const u16* A, int64_t lda, const uint8_t* B, int64_t ldb, const float* s_w, int G,
                      int gsize, const void* bias, int bias_dt, u16* C, int64_t ldc, int M, int N, int K,
-                     bool mfma_ok, bool big_ok, hipStream_t st) {
+                     bool mfma_ok, bool big_ok, void* ws, int64_t ws_bytes, hipStream_t st) {
+  if (big_ok) {
+    const MidPlan p = w16_plan(M, N, K, w16_max_splits(M, N, ws, ws_bytes));
+    if (p.S > 0) return launch_w16_mid<DT>(A, lda, B, ldb, s_w, G, bias, bias_dt, C, ldc, M, N, K, ws, false, p, st);
+  }
   if (mfma_ok) {
     if (M > 128 && big_ok) return launch_w4a16_big<DT>(A, lda, B, ldb, s_w, G, bias, bias_dt, C, ldc, M, N, K, st);
     if (M > 128) {
@@ -445,9 +485,24 @@ __global__ void w4a16_stage_s_kernel(const float* __restrict__ S, float* __restr
 
 extern "C" {
 
+int64_t ic_gemm_w4a16_splitk_bytes(int64_t M, int64_t N, int64_t K, int64_t num_groups) {
+  if (M <= IC_GEMV_MAX_M || N <= 0 || K <= 0 || K % 64 != 0 || num_groups < 1 || K % num_groups != 0 || (N & 7) != 0)
+    return 0;
+  if ((num_groups > 1 && (K / num_groups) % 64 != 0) || M * N > (1LL << 31)) return 0;
+  const MidPlan p = w16_plan(M, N, K, kW16MaxSplits);
+  return p.S > 1 ? (int64_t)p.S * M * N * 4 : 0;
+}
+
 int ic_gemm_w4a16(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_packed,
                   int64_t N, int64_t ldw, const float* s_w, int64_t num_groups, const void* bias,
                   int bias_dtype, void* out, int64_t ldo, void* stream) {
+  return ic_gemm_w4a16_ws(x, dtype, M, K, ldx, w_packed, N, ldw, s_w, num_groups, bias, bias_dtype, out, ldo, nullptr,
+                          0, stream);
+}
+
+int ic_gemm_w4a16_ws(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_packed,
+                     int64_t N, int64_t ldw, const float* s_w, int64_t num_groups, const void* bias,
+                     int bias_dtype, void* out, int64_t ldo, void* workspace, int64_t workspace_bytes, void* stream) {
   const char* who = "ic_gemm_w4a16";
   if (dtype != IC_DTYPE_F16 && dtype != IC_DTYPE_BF16)
     return ic_set_error(IC_ERR_INVALID_ARG, "%s: activation dtype must be f16/bf16", who);
@@ -476,9 +531,11 @@ int ic_gemm_w4a16(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, c
   hipStream_t st = (hipStream_t)stream;
   hipError_t e = dtype == IC_DTYPE_F16
                      ? run_w4a16<IC_DTYPE_F16>((const u16*)x, ldx, w_packed, ldw, s_w, G, gsize, bias, bias_dtype,
-                                               (u16*)out, ldo, (int)M, (int)N, (int)K, mfma_ok, big_ok, st)
+                                               (u16*)out, ldo, (int)M, (int)N, (int)K, mfma_ok, big_ok, workspace,
+                                               workspace_bytes, st)
                      : run_w4a16<IC_DTYPE_BF16>((const u16*)x, ldx, w_packed, ldw, s_w, G, gsize, bias, bias_dtype,
-                                                (u16*)out, ldo, (int)M, (int)N, (int)K, mfma_ok, big_ok, st);
+                                                (u16*)out, ldo, (int)M, (int)N, (int)K, mfma_ok, big_ok, workspace,
+                                               workspace_bytes, st);
   if (e != hipSuccess) return ic_set_error(IC_ERR_LAUNCH, "%s: %s", who, hipGetErrorString(e));
   return IC_OK;
 }
@@ -506,6 +563,13 @@ int ic_w4a16_stage_layout(const uint8_t* w_packed, int64_t N, int64_t K, int64_t
 int ic_gemm_w4a16_staged(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_staged,
                          int64_t N, const float* s_staged, int64_t num_groups, const void* bias, int bias_dtype,
                          void* out, int64_t ldo, void* stream) {
+  return ic_gemm_w4a16_staged_ws(x, dtype, M, K, ldx, w_staged, N, s_staged, num_groups, bias, bias_dtype, out, ldo,
+                                 nullptr, 0, stream);
+}
+
+int ic_gemm_w4a16_staged_ws(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_staged,
+                            int64_t N, const float* s_staged, int64_t num_groups, const void* bias, int bias_dtype,
+                            void* out, int64_t ldo, void* workspace, int64_t workspace_bytes, void* stream) {
   const char* who = "ic_gemm_w4a16_staged";
   if (dtype != IC_DTYPE_F16 && dtype != IC_DTYPE_BF16)
     return ic_set_error(IC_ERR_INVALID_ARG, "%s: activation dtype must be f16/bf16", who);
@@ -529,7 +593,16 @@ int ic_gemm_w4a16_staged(const void* x, int dtype, int64_t M, int64_t K, int64_t
                         "other shapes take ic_gemm_w4a16",
                         who, (long long)M, (long long)N, (long long)K, (long long)num_groups);
   hipStream_t st = (hipStream_t)stream;
-  hipError_t e = dtype == IC_DTYPE_F16
+  const MidPlan p = w16_plan(M, N, K, w16_max_splits(M, N, workspace, workspace_bytes));
+  hipError_t e;
+  if (p.S > 0)
+    e = dtype == IC_DTYPE_F16
+            ? launch_w16_mid<IC_DTYPE_F16>((const u16*)x, ldx, w_staged, N * 32, s_staged, G, bias, bias_dtype,
+                                           (u16*)out, ldo, (int)M, (int)N, (int)K, workspace, true, p, st)
+            : launch_w16_mid<IC_DTYPE_BF16>((const u16*)x, ldx, w_staged, N * 32, s_staged, G, bias, bias_dtype,
+                                            (u16*)out, ldo, (int)M, (int)N, (int)K, workspace, true, p, st);
+  else
+    e = dtype == IC_DTYPE_F16
                      ? launch_w4a16_big<IC_DTYPE_F16, true>((const u16*)x, ldx, w_staged, N * 32, s_staged, G, bias,
                                                             bias_dtype, (u16*)out, ldo, (int)M, (int)N, (int)K, st)
                      : launch_w4a16_big<IC_DTYPE_BF16, true>((const u16*)x, ldx, w_staged, N * 32, s_staged, G, bias,

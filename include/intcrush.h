@@ -175,8 +175,10 @@ int ic_gemm_w4a8(const int8_t* xq, int64_t M, int64_t K, int64_t ldx, const uint
  * second kernel adds them in slice order and applies the epilogue.  Per-row
  * scale outputs are bit-identical to the unsplit GEMM; grouped outputs differ
  * only in the order of the fp32 additions.  ic_gemm_splitk_bytes returns the
- * workspace the launch will use (0: no split; then workspace may be null);
- * a smaller workspace than that runs the unsplit GEMM.  The library itself
+ * most workspace a launch of that shape uses (0: no split; then workspace may
+ * be null); a smaller workspace than that runs on fewer slices or unsplit.
+ * Launches with 16-bit, 16-byte aligned outputs may take small tiles instead,
+ * in fewer slices or none.  The library itself
  * never allocates.
  */
 int64_t ic_gemm_splitk_bytes(int64_t M, int64_t N, int64_t K, int64_t num_groups, int int4);
@@ -335,6 +337,22 @@ int ic_w4a16_stage_layout(const uint8_t* w_packed, int64_t N, int64_t K, int64_t
 int ic_gemm_w4a16_staged(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_staged,
                          int64_t N, const float* s_staged, int64_t num_groups, const void* bias, int bias_dtype,
                          void* out, int64_t ldo, void* stream);
+
+/*
+ * Split-K forms of ic_gemm_w4a16 / ic_gemm_w4a16_staged, for launches whose
+ * output tiles leave most CUs idle: K slices run in parallel, their fp32 sums
+ * go to the caller's workspace and a second kernel adds them in slice order.
+ * ic_gemm_w4a16_splitk_bytes is the workspace such a launch uses (0: no
+ * split); with less, or none, it runs on fewer slices or unsplit, as the
+ * entry points without a workspace do.  No reference counterpart.
+ */
+int64_t ic_gemm_w4a16_splitk_bytes(int64_t M, int64_t N, int64_t K, int64_t num_groups);
+int ic_gemm_w4a16_ws(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_packed,
+                     int64_t N, int64_t ldw, const float* s_w, int64_t num_groups, const void* bias,
+                     int bias_dtype, void* out, int64_t ldo, void* workspace, int64_t workspace_bytes, void* stream);
+int ic_gemm_w4a16_staged_ws(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_staged,
+                            int64_t N, const float* s_staged, int64_t num_groups, const void* bias, int bias_dtype,
+                            void* out, int64_t ldo, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * Small-batch GEMV forms (1 <= M <= IC_GEMV_MAX_M tokens, K a multiple of 128
