@@ -112,6 +112,7 @@ SIGNATURES: dict[str, tuple[list, object]] = {
 }
 
 _lib = None
+_max_fused_row = 0  # ic_max_fused_row() of the loaded library
 
 
 def _load():
@@ -125,11 +126,12 @@ def _load():
 
 def load_library(reload: bool = False):
     """(Re)load the shared library and refresh the availability flags."""
-    global _lib, LOAD_ERROR
+    global _lib, _max_fused_row, LOAD_ERROR
     if _lib is not None and not reload:
         return _lib
     try:
         _lib = _load()
+        _max_fused_row = int(_lib.ic_max_fused_row())
         LOAD_ERROR = None
         log.info("[INT-Crush] HIP kernels loaded: %s", _lib.ic_version().decode())
     except (OSError, AttributeError) as exc:
@@ -184,6 +186,49 @@ def _call(name: str, *args) -> None:
         raise RuntimeError(f"[INT-Crush] {name} failed ({rc}): {lib().ic_last_error().decode()}")
 
 
+# The launches below are what one linear costs on the host: a pass over one to a
+# few hundred tokens took ~17 us of Python for each of its two calls against
+# 5 to 15 us on the GPU.  Hence raw addresses and stream handles instead of ctypes and
+# Stream objects, a device guard only off the current device, and no tensor
+# operations on operands that already have the form the kernels read.
+def _addr(t: torch.Tensor | None):
+    return None if t is None else t.data_ptr()
+
+
+_get_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                      lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
+def _launch(name: str, t: torch.Tensor, *args) -> None:
+    """_call on t's device, with the current stream of that device appended."""
+    fn = getattr(lib(), name)
+    index = t.get_device()
+    if _get_device() == index:
+        rc = fn(*args, _raw_stream(index))
+    else:
+        with torch.cuda.device(index):
+            rc = fn(*args, _raw_stream(index))
+    if rc != 0:
+        raise RuntimeError(f"[INT-Crush] {name} failed ({rc}): {lib().ic_last_error().decode()}")
+
+
+def _f32_flat(t: torch.Tensor) -> torch.Tensor:
+    """The values of t as contiguous float32, in order (its shape is not read)."""
+    if t.dtype is torch.float32 and t.is_contiguous():
+        return t
+    return t.detach().reshape(-1).to(torch.float32).contiguous()
+
+
+def _group_scales(s_w: torch.Tensor, N: int) -> tuple[torch.Tensor, int]:
+    """Weight scales [N, G] (or [N]) as contiguous float32, and G."""
+    n = s_w.numel()
+    if s_w.dtype is torch.float32 and N > 0 and n > 0 and n % N == 0 and s_w.is_contiguous():
+        return s_w, n // N
+    sw = s_w.detach().reshape(N, -1).to(torch.float32).contiguous()
+    return sw, sw.shape[1]
+
+
 def _dt(t: torch.dtype, who: str) -> int:
     if t not in _DT_CODE:
         raise TypeError(f"{who}: unsupported dtype {t} (expected float16, bfloat16 or float32)")
@@ -198,6 +243,8 @@ def _need_cuda(*tensors: torch.Tensor | None) -> None:
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
     """2-D view with unit column stride (copy only when required)."""
+    if t.dim() == 2 and t.stride(1) == 1 and (t.shape[0] <= 1 or t.stride(0) >= t.shape[1]):
+        return t
     t2 = t.reshape(-1, t.shape[-1])
     if t2.stride(-1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < t2.shape[1]):
         t2 = t2.contiguous()
@@ -284,25 +331,25 @@ def rotate_quantize(x: torch.Tensor, *, rot_size: int = 0, w_in: int | None = No
     x2 = _rows(x)
     M, K_in = x2.shape
     R, K_w, dt = _prep_shape(x2, rot_size, w_in, smoothrot, perm, smooth, "rotate_quantize")
-    s_a = _alloc_or_reuse((M,), torch.float32, x2.device, s_a_out)
-    q = _alloc_or_reuse((M, K_w), torch.int8, x2.device, x_int8_out)
-    with torch.cuda.device(x2.device):
-        if K_w <= _fused_limit(dt):
-            _call("ic_rotate_quantize", _ptr(x2), dt, M, K_in, x2.stride(0),
-                  _ptr(smoothrot.rcp) if smoothrot else None, _ptr(smoothrot.fdt) if smoothrot else None,
-                  R, K_w, _ptr(perm), _ptr(smooth.rcp) if smooth else None,
-                  _ptr(smooth.fdt) if smooth else None, _ptr(q), q.stride(0), _ptr(s_a), _stream(x2))
-        else:
+    device = x2.device
+    s_a = _alloc_or_reuse((M,), torch.float32, device, s_a_out)
+    q = _alloc_or_reuse((M, K_w), torch.int8, device, x_int8_out)
+    sm_rcp, sm_f = (smooth.rcp.data_ptr(), smooth.fdt.data_ptr()) if smooth else (None, None)
+    if K_w <= _fused_limit(dt):
+        sr_rcp, sr_f = (smoothrot.rcp.data_ptr(), smoothrot.fdt.data_ptr()) if smoothrot else (None, None)
+        _launch("ic_rotate_quantize", x2, x2.data_ptr(), dt, M, K_in, x2.stride(0), sr_rcp, sr_f, R, K_w, _addr(perm),
+                sm_rcp, sm_f, q.data_ptr(), q.stride(0), s_a.data_ptr())
+    else:
+        with torch.cuda.device(device):
             y = _rotate_wide(x2, R, smoothrot, dt)
-            _call("ic_permute_quantize", _ptr(y), dt, M, y.shape[1], y.stride(0), K_w, _ptr(perm),
-                  _ptr(smooth.rcp) if smooth else None, _ptr(smooth.fdt) if smooth else None,
-                  _ptr(q), q.stride(0), _ptr(s_a), None, 0, _stream(y))
+            _launch("ic_permute_quantize", y, y.data_ptr(), dt, M, y.shape[1], y.stride(0), K_w, _addr(perm), sm_rcp,
+                    sm_f, q.data_ptr(), q.stride(0), s_a.data_ptr(), None, 0)
     return q, s_a
 
 
 def _fused_limit(dt: int) -> int:
     """Widest row the single-pass prep kernels hold."""
-    return lib().ic_max_fused_row() // (2 if dt == IC_DTYPE_F32 else 1)
+    return _max_fused_row // (2 if dt == IC_DTYPE_F32 else 1)
 
 
 def _rotate_wide(x2: torch.Tensor, R: int, smoothrot: PreparedFactors | None, dt: int) -> torch.Tensor:
@@ -341,17 +388,16 @@ def prepare_activation(x: torch.Tensor, *, rot_size: int = 0, w_in: int | None =
     if perm is not None and (perm.dtype != torch.int32 or perm.numel() != K_w):
         raise ValueError("perm must be an int32 device tensor of length w_in (see prepare_perm)")
     y = _alloc_or_reuse((M, K_w), x2.dtype, x2.device, out)
-    with torch.cuda.device(x2.device):
-        if K_w <= _fused_limit(dt):
-            _call("ic_prepare_activation", _ptr(x2), dt, M, K_in, x2.stride(0),
-                  _ptr(smoothrot.rcp) if smoothrot else None, _ptr(smoothrot.fdt) if smoothrot else None,
-                  R, K_w, _ptr(perm), _ptr(smooth.rcp) if smooth else None,
-                  _ptr(smooth.fdt) if smooth else None, _ptr(y), y.stride(0), _stream(x2))
-        else:
+    sm_rcp, sm_f = (smooth.rcp.data_ptr(), smooth.fdt.data_ptr()) if smooth else (None, None)
+    if K_w <= _fused_limit(dt):
+        sr_rcp, sr_f = (smoothrot.rcp.data_ptr(), smoothrot.fdt.data_ptr()) if smoothrot else (None, None)
+        _launch("ic_prepare_activation", x2, x2.data_ptr(), dt, M, K_in, x2.stride(0), sr_rcp, sr_f, R, K_w,
+                _addr(perm), sm_rcp, sm_f, y.data_ptr(), y.stride(0))
+    else:
+        with torch.cuda.device(x2.device):
             yr = _rotate_wide(x2, R, smoothrot, dt)
-            _call("ic_permute_quantize", _ptr(yr), dt, M, yr.shape[1], yr.stride(0), K_w, _ptr(perm),
-                  _ptr(smooth.rcp) if smooth else None, _ptr(smooth.fdt) if smooth else None,
-                  None, 0, None, _ptr(y), y.stride(0), _stream(yr))
+            _launch("ic_permute_quantize", yr, yr.data_ptr(), dt, M, yr.shape[1], yr.stride(0), K_w, _addr(perm),
+                    sm_rcp, sm_f, None, 0, None, y.data_ptr(), y.stride(0))
     return y
 
 
@@ -378,9 +424,8 @@ def dynamic_quantize_activation(x: torch.Tensor, s_a_out: torch.Tensor | None = 
         x2 = _rows(x2)
         s = _alloc_or_reuse((M,), torch.float32, x2.device, s_a_out)
         q = _alloc_or_reuse((M, K), torch.int8, x2.device, x_int8_out)
-        with torch.cuda.device(x2.device):
-            _call("ic_dynamic_quantize", _ptr(x2), _dt(x2.dtype, "dynamic_quantize_activation"), M, K,
-                  x2.stride(0), _ptr(q), q.stride(0), _ptr(s), _stream(x2))
+        _launch("ic_dynamic_quantize", x2, x2.data_ptr(), _dt(x2.dtype, "dynamic_quantize_activation"), M, K,
+                x2.stride(0), q.data_ptr(), q.stride(0), s.data_ptr())
     if orig_shape != x2.shape:
         q = q.reshape(orig_shape)
         s = s.reshape(*orig_shape[:-1])
@@ -394,10 +439,11 @@ IC_NORM_LAYER, IC_NORM_RMS, IC_SOFTMAX = 1, 2, 3
 def _f32_vec(t: torch.Tensor | None, K: int, who: str, device) -> torch.Tensor | None:
     if t is None:
         return None
-    v = t.detach().reshape(-1)
-    if v.numel() != K:
-        raise ValueError(f"{who} has {v.numel()} entries, expected {K}")
-    return v.to(device=device, dtype=torch.float32).contiguous()
+    if t.numel() != K:
+        raise ValueError(f"{who} has {t.numel()} entries, expected {K}")
+    if t.dtype is torch.float32 and t.device == device and t.is_contiguous():
+        return t
+    return t.detach().reshape(-1).to(device=device, dtype=torch.float32).contiguous()
 
 
 def _norm_quantize(x: torch.Tensor, kind: int, gamma, beta, eps: float, s_a_out, x_int8_out, who: str):
@@ -408,9 +454,8 @@ def _norm_quantize(x: torch.Tensor, kind: int, gamma, beta, eps: float, s_a_out,
     q = _alloc_or_reuse((M, K), torch.int8, x2.device, x_int8_out)
     g = _f32_vec(gamma, K, "gamma", x2.device)
     b = _f32_vec(beta, K, "beta", x2.device)
-    with torch.cuda.device(x2.device):
-        _call("ic_norm_quantize", _ptr(x2), _dt(x2.dtype, who), M, K, x2.stride(0), kind, _ptr(g), _ptr(b),
-              float(eps), _ptr(q), q.stride(0), _ptr(s), _stream(x2))
+    _launch("ic_norm_quantize", x2, x2.data_ptr(), _dt(x2.dtype, who), M, K, x2.stride(0), kind, _addr(g), _addr(b),
+            float(eps), q.data_ptr(), q.stride(0), s.data_ptr())
     if orig_shape != x2.shape:
         q = q.reshape(orig_shape)
         s = s.reshape(*orig_shape[:-1])
@@ -450,10 +495,9 @@ def norm_rotate_quantize(x: torch.Tensor, *, norm: str = "layer", weight: torch.
     b = _f32_vec(bias, K_in, "bias", x2.device)
     s_a = _alloc_or_reuse((M,), torch.float32, x2.device, s_a_out)
     q = _alloc_or_reuse((M, K_w), torch.int8, x2.device, x_int8_out)
-    with torch.cuda.device(x2.device):
-        _call("ic_norm_rotate_quantize", _ptr(x2), dt, M, K_in, x2.stride(0), kind, _ptr(w), _ptr(b), float(eps),
-              _ptr(smoothrot.rcp) if smoothrot else None, _ptr(smoothrot.fdt) if smoothrot else None, R, K_w,
-              _ptr(perm), _ptr(q), q.stride(0), _ptr(s_a), _stream(x2))
+    sr_rcp, sr_f = (smoothrot.rcp.data_ptr(), smoothrot.fdt.data_ptr()) if smoothrot else (None, None)
+    _launch("ic_norm_rotate_quantize", x2, x2.data_ptr(), dt, M, K_in, x2.stride(0), kind, _addr(w), _addr(b),
+            float(eps), sr_rcp, sr_f, R, K_w, _addr(perm), q.data_ptr(), q.stride(0), s_a.data_ptr())
     return q, s_a
 
 
@@ -505,11 +549,10 @@ def fused_softmax_quantize(x: torch.Tensor, s_a_out: torch.Tensor | None = None,
 def _bias_args(bias: torch.Tensor | None, N: int):
     if bias is None:
         return None, 0, None
-    b = bias.detach().reshape(-1)
-    if b.numel() != N:
-        raise ValueError(f"bias has {b.numel()} entries, expected {N}")
-    b = b.contiguous()
-    return _ptr(b), _dt(b.dtype, "bias"), b
+    if bias.numel() != N:
+        raise ValueError(f"bias has {bias.numel()} entries, expected {N}")
+    b = bias if bias.is_contiguous() else bias.detach().reshape(-1).contiguous()
+    return b.data_ptr(), _dt(b.dtype, "bias"), b
 
 
 def _out_buffer(out, M, N, out_dtype, device):
@@ -520,11 +563,16 @@ def _out_buffer(out, M, N, out_dtype, device):
     return torch.empty((M, N), dtype=out_dtype, device=device)
 
 
+GEMV_MAX_M = 16  # IC_GEMV_MAX_M
+
+
 def _splitk_workspace(M: int, N: int, K: int, G: int, int4: bool, device) -> tuple[torch.Tensor | None, int]:
     """Workspace for the split-K form of the GEMM when the library plans one
     (small M: too few output tiles to occupy the GPU); (None, 0) otherwise.
     Allocated from torch's caching allocator, so it is graph-capture safe."""
-    nb = int(lib().ic_gemm_splitk_bytes(M, N, K, G, 1 if int4 else 0))
+    if M <= GEMV_MAX_M:
+        return None, 0  # as ic_gemm_splitk_bytes answers for these
+    nb = lib().ic_gemm_splitk_bytes(M, N, K, G, 1 if int4 else 0)
     if nb <= 0:
         return None, 0
     return torch.empty(nb, dtype=torch.uint8, device=device), nb
@@ -532,7 +580,9 @@ def _splitk_workspace(M: int, N: int, K: int, G: int, int4: bool, device) -> tup
 
 def _w16_workspace(M: int, N: int, K: int, G: int, device) -> tuple[torch.Tensor | None, int]:
     """The same for the W4A16 GEMM (ic_gemm_w4a16_splitk_bytes)."""
-    nb = int(lib().ic_gemm_w4a16_splitk_bytes(M, N, K, G))
+    if M <= GEMV_MAX_M:
+        return None, 0
+    nb = lib().ic_gemm_w4a16_splitk_bytes(M, N, K, G)
     if nb <= 0:
         return None, 0
     return torch.empty(nb, dtype=torch.uint8, device=device), nb
@@ -580,19 +630,19 @@ def fused_int8_gemm_dequant(x_int8: torch.Tensor, w_int8: torch.Tensor, s_w: tor
     assert K == K_w, f"K mismatch: {K} vs {K_w}"
     xq = _rows(x_int8)
     w = _rows(w_int8)
-    sw = s_w.detach().reshape(-1).to(torch.float32).contiguous()
+    sw = _f32_flat(s_w)
     if sw.numel() != N:
         raise ValueError(f"s_w must hold one scale per output channel ({N}), got {sw.numel()}")
-    sa = s_a.detach().reshape(-1).to(torch.float32).contiguous()
+    sa = _f32_flat(s_a)
     bp, bdt, _keep = _bias_args(bias, N)
     act, rp, rdt, ldr, _rkeep = _epilogue_args(activation, residual, M, N)
-    c = _out_buffer(out, M, N, out_dtype, x_int8.device)
-    _warn_if_scalar_gemm("fused_int8_gemm_dequant", K, 1, xq, w)
-    with torch.cuda.device(xq.device):
-        ws, nb = _splitk_workspace(M, N, K, 1, False, xq.device)
-        _call("ic_gemm_w8a8_ex", _ptr(xq), M, K, xq.stride(0), _ptr(w), N, w.stride(0), _ptr(sa),
-              _ptr(sw), bp, bdt, act, rp, rdt, ldr, _ptr(c), _dt(c.dtype, "out"), c.stride(0), _ptr(ws), nb,
-              _stream(xq))
+    device = xq.device
+    c = _out_buffer(out, M, N, out_dtype, device)
+    xp, ldx, wp, ldw = xq.data_ptr(), xq.stride(0), w.data_ptr(), w.stride(0)
+    _warn_if_scalar_gemm("fused_int8_gemm_dequant", K, 1, xp | ldx | wp | ldw)
+    ws, nb = _splitk_workspace(M, N, K, 1, False, device)
+    _launch("ic_gemm_w8a8_ex", xq, xp, M, K, ldx, wp, N, ldw, sa.data_ptr(), sw.data_ptr(), bp, bdt, act, rp, rdt, ldr,
+            c.data_ptr(), _dt(c.dtype, "out"), c.stride(0), _addr(ws), nb)
     return c
 
 
@@ -636,19 +686,19 @@ def fused_w4a8_gemm_dequant(x_int8, w_int8, s_w, s_a, bias=None, out_dtype=torch
 _SCALAR_WARNED: set = set()
 
 
-def _warn_if_scalar_gemm(who: str, K: int, G: int, *tensors: torch.Tensor, out64: bool = False) -> None:
+def _warn_if_scalar_gemm(who: str, K: int, G: int, align: int, out64: bool = False) -> None:
     """The INT8 / W4A8 GEMMs run MFMA tiles only for K a multiple of 128,
     group sizes that are multiples of 128 (W4A8 also odd multiples of 64 or
     of 32 when out64: a 16-bit output whose rows and residual suit the
     288 x 192 tile's staged stores) and 16-byte aligned operands and row
-    strides; anything else takes the scalar kernel (one thread per output,
-    ~100x slower).  Log that once per shape instead of running it silently."""
+    strides (align: their addresses and byte strides, or-ed); anything else
+    takes the scalar kernel (one thread per output, ~100x slower).  Log that
+    once per shape instead of running it silently."""
     gs = K // G
-    ok = K % 128 == 0 and (G == 1 or gs % 128 == 0 or (out64 and gs % 32 == 0))
-    for t in tensors:
-        ok = ok and t.data_ptr() % 16 == 0 and (t.dim() < 2 or (t.stride(0) * t.element_size()) % 16 == 0)
+    if K % 128 == 0 and (G == 1 or gs % 128 == 0 or (out64 and gs % 32 == 0)) and align & 15 == 0:
+        return
     key = (who, K, G)
-    if not ok and key not in _SCALAR_WARNED:
+    if key not in _SCALAR_WARNED:
         _SCALAR_WARNED.add(key)
         log.warning("[INT-Crush] %s: K=%d, group size %d or operand alignment has no MFMA tiling; "
                     "running the scalar fallback kernel (about 100x slower)", who, K, gs)
@@ -693,22 +743,21 @@ def gemm_w4a8(x_int8: torch.Tensor, w_packed: torch.Tensor, s_w: torch.Tensor, s
     N = w_packed.shape[0]
     assert w_packed.shape[1] * 2 >= K, f"packed weight too narrow for K={K}"
     w = _rows(w_packed)
-    sw = s_w.detach().reshape(N, -1).to(torch.float32).contiguous()
-    G = sw.shape[1]
+    sw, G = _group_scales(s_w, N)
     if K % G:
         raise ValueError(f"K={K} is not a multiple of the {G} scale groups")
-    sa = s_a.detach().reshape(-1).to(torch.float32).contiguous()
+    sa = _f32_flat(s_a)
     bp, bdt, _keep = _bias_args(bias, N)
     act, rp, rdt, ldr, _rkeep = _epilogue_args(activation, residual, M, N)
-    c = _out_buffer(out, M, N, out_dtype, xq.device)
-    out64 = (c.dtype != torch.float32 and N % 8 == 0 and c.data_ptr() % 16 == 0 and c.stride(0) % 8 == 0
+    device = xq.device
+    c = _out_buffer(out, M, N, out_dtype, device)
+    xp, ldx, wp, ldw, cp, ldc = xq.data_ptr(), xq.stride(0), w.data_ptr(), w.stride(0), c.data_ptr(), c.stride(0)
+    out64 = (c.dtype != torch.float32 and N % 8 == 0 and cp % 16 == 0 and ldc % 8 == 0
              and (rp is None or (rdt != 2 and (rp.value or 0) % 16 == 0 and ldr % 8 == 0)))
-    _warn_if_scalar_gemm("gemm_w4a8", K, G, xq, w, out64=out64)
-    with torch.cuda.device(xq.device):
-        ws, nb = _splitk_workspace(M, N, K, G, True, xq.device)
-        _call("ic_gemm_w4a8_kil_ex" if kil else "ic_gemm_w4a8_ex", _ptr(xq), M, K, xq.stride(0), _ptr(w), N,
-              w.stride(0), _ptr(sw), G, _ptr(sa), bp, bdt, act, rp, rdt, ldr, _ptr(c), _dt(c.dtype, "out"),
-              c.stride(0), _ptr(ws), nb, _stream(xq))
+    _warn_if_scalar_gemm("gemm_w4a8", K, G, xp | ldx | wp | ldw, out64)
+    ws, nb = _splitk_workspace(M, N, K, G, True, device)
+    _launch("ic_gemm_w4a8_kil_ex" if kil else "ic_gemm_w4a8_ex", xq, xp, M, K, ldx, wp, N, ldw, sw.data_ptr(), G,
+            sa.data_ptr(), bp, bdt, act, rp, rdt, ldr, cp, _dt(c.dtype, "out"), ldc, _addr(ws), nb)
     return c
 
 def w4a8_unpacked_pays(M: int, N: int, K: int, G: int, device=None) -> bool:
@@ -743,20 +792,19 @@ def gemm_w4a8_unpacked(x_int8: torch.Tensor, w_int8: torch.Tensor, s_w: torch.Te
     N = w_int8.shape[0]
     assert w_int8.shape[1] >= K, f"unpacked weight too narrow for K={K}"
     w = _rows(w_int8)
-    sw = s_w.detach().reshape(N, -1).to(torch.float32).contiguous()
-    G = sw.shape[1]
+    sw, G = _group_scales(s_w, N)
     if K % G:
         raise ValueError(f"K={K} is not a multiple of the {G} scale groups")
-    sa = s_a.detach().reshape(-1).to(torch.float32).contiguous()
+    sa = _f32_flat(s_a)
     bp, bdt, _keep = _bias_args(bias, N)
     act, rp, rdt, ldr, _rkeep = _epilogue_args(activation, residual, M, N)
-    c = _out_buffer(out, M, N, out_dtype, xq.device)
-    _warn_if_scalar_gemm("gemm_w4a8_unpacked", K, G, xq, w)
-    with torch.cuda.device(xq.device):
-        ws, nb = _splitk_workspace(M, N, K, G, False, xq.device)
-        _call("ic_gemm_w4a8_unpacked_ex", _ptr(xq), M, K, xq.stride(0), _ptr(w), N, w.stride(0), _ptr(sw), G,
-              _ptr(sa), bp, bdt, act, rp, rdt, ldr, _ptr(c), _dt(c.dtype, "out"), c.stride(0), _ptr(ws), nb,
-              _stream(xq))
+    device = xq.device
+    c = _out_buffer(out, M, N, out_dtype, device)
+    xp, ldx, wp, ldw = xq.data_ptr(), xq.stride(0), w.data_ptr(), w.stride(0)
+    _warn_if_scalar_gemm("gemm_w4a8_unpacked", K, G, xp | ldx | wp | ldw)
+    ws, nb = _splitk_workspace(M, N, K, G, False, device)
+    _launch("ic_gemm_w4a8_unpacked_ex", xq, xp, M, K, ldx, wp, N, ldw, sw.data_ptr(), G, sa.data_ptr(), bp, bdt, act,
+            rp, rdt, ldr, c.data_ptr(), _dt(c.dtype, "out"), c.stride(0), _addr(ws), nb)
     return c
 
 
@@ -891,8 +939,7 @@ def gemm_w4a16(x: torch.Tensor, w_packed: torch.Tensor, s_w: torch.Tensor,
     N = w_packed.shape[0]
     assert w_packed.shape[1] * 2 >= K, f"packed weight too narrow for K={K}"
     w = _rows(w_packed)
-    sw = s_w.detach().reshape(N, -1).to(torch.float32).contiguous()
-    G = sw.shape[1]
+    sw, G = _group_scales(s_w, N)
     if K % G:
         raise ValueError(f"K={K} is not a multiple of the {G} scale groups")
     dt = _dt(x2.dtype, "gemm_w4a16")
@@ -900,10 +947,9 @@ def gemm_w4a16(x: torch.Tensor, w_packed: torch.Tensor, s_w: torch.Tensor,
         raise TypeError("gemm_w4a16 needs float16 or bfloat16 activations")
     bp, bdt, _keep = _bias_args(bias, N)
     c = _out_buffer(out, M, N, x2.dtype, x2.device)
-    with torch.cuda.device(x2.device):
-        ws, nb = _w16_workspace(M, N, K, G, x2.device)
-        _call("ic_gemm_w4a16_ws", _ptr(x2), dt, M, K, x2.stride(0), _ptr(w), N, w.stride(0), _ptr(sw), G,
-              bp, bdt, _ptr(c), c.stride(0), _ptr(ws), nb, _stream(x2))
+    ws, nb = _w16_workspace(M, N, K, G, x2.device)
+    _launch("ic_gemm_w4a16_ws", x2, x2.data_ptr(), dt, M, K, x2.stride(0), w.data_ptr(), N, w.stride(0), sw.data_ptr(),
+            G, bp, bdt, c.data_ptr(), c.stride(0), _addr(ws), nb)
     return c
 
 
@@ -949,23 +995,21 @@ def gemm_w4a16_staged(x: torch.Tensor, w_staged: torch.Tensor, s_staged: torch.T
     S, N, _ = w_staged.shape
     if 64 * S != K:
         raise ValueError(f"staged weights cover K={64 * S}, activations K={K}")
-    ss = s_staged.detach().to(torch.float32).contiguous()
-    G = ss.shape[0]
+    G = s_staged.shape[0]
+    ss = _f32_flat(s_staged)
+    wst = w_staged if w_staged.is_contiguous() else w_staged.contiguous()
     dt = _dt(x2.dtype, "gemm_w4a16_staged")
     if dt == IC_DTYPE_F32:
         raise TypeError("gemm_w4a16_staged needs float16 or bfloat16 activations")
     bp, bdt, _keep = _bias_args(bias, N)
     c = _out_buffer(out, M, N, x2.dtype, x2.device)
-    with torch.cuda.device(x2.device):
-        ws, nb = _w16_workspace(M, N, K, G, x2.device)
-        _call("ic_gemm_w4a16_staged_ws", _ptr(x2), dt, M, K, x2.stride(0), _ptr(w_staged.contiguous()), N, _ptr(ss),
-              G, bp, bdt, _ptr(c), c.stride(0), _ptr(ws), nb, _stream(x2))
+    ws, nb = _w16_workspace(M, N, K, G, x2.device)
+    _launch("ic_gemm_w4a16_staged_ws", x2, x2.data_ptr(), dt, M, K, x2.stride(0), wst.data_ptr(), N, ss.data_ptr(), G,
+            bp, bdt, c.data_ptr(), c.stride(0), _addr(ws), nb)
     return c
 
 
 # ── small-batch GEMV (M <= 16; the GEMM callables route there by themselves) ──
-GEMV_MAX_M = 16
-
 
 def gemv(x: torch.Tensor, w: torch.Tensor, s_w: torch.Tensor, s_a: torch.Tensor | None = None,
          bias: torch.Tensor | None = None, out_dtype: torch.dtype | None = None, *,
