@@ -124,6 +124,19 @@ IC_DEV float rto24(double y) {
   return (float)__longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
+// Round-to-odd to 21 significant bits (the high word, its lowest bit set if any
+// of the low word is): two cheap instructions and an exact conversion.  In f32's
+// normal range RN_dt(rto_hi(y)) == RN_dt(y) for any 16-bit type (21 >= p + 2
+// with p <= 11, f16 subnormals have fewer bits still).
+IC_DEV float rto_hi(double y) {
+  const uint64_t b = (uint64_t)__double_as_longlong(y);
+  const uint32_t lo = (uint32_t)b;
+  uint32_t any;  // min(lo, 1), which the compiler turns into a compare and a select
+  asm("v_min_u32 %0, 1, %1" : "=v"(any) : "v"(lo));
+  const uint32_t hi = (uint32_t)(b >> 32) | any;
+  return (float)__longlong_as_double((long long)((uint64_t)hi << 32));
+}
+
 // RN of an fp64 value to DT, returned as the f32 holding that exact value.
 template <int DT> IC_DEV float round_f64_to_dt(double y) {
   if constexpr (DT == IC_DTYPE_F32) return (float)y;

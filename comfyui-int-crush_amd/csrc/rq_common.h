@@ -121,16 +121,6 @@ template <int TILE> constexpr int tslot_doubles() { return TILE + 2 * (TILE / 16
 IC_DEV int rbaddr(int p) { return p + 16 * (p >> 8); }
 template <int NT, int TILE> constexpr int rowbuf_len() { return NT * TILE + 16 * (NT * TILE / 256); }
 
-// RN_dt(y) of an fp64 value through RN32: exact unless RN32(y) is itself a
-// rounding boundary of DT (a midpoint between neighbours, including the
-// overflow threshold) or lies below DT's normal range.  Boundary test on the
-// f32 bits: the bits below DT's precision are exactly 100...0.
-template <int DT> IC_DEV uint32_t rn32_boundary_key(float z) {
-  const uint32_t w = __float_as_uint(z);
-  if constexpr (DT == IC_DTYPE_F16) return (w ^ 0x1000u) & 0x1fffu;  // zero iff (w & 0x1fff) == 0x1000
-  else return (w ^ 0x8000u) & 0xffffu;
-}
-
 constexpr int kFastMaxTiles = 4;  // fast path: K_w <= 16384
 
 // ---- bf16 flush of values far below their Hadamard block's maximum.

@@ -58,13 +58,40 @@ IC_DEV v4u quant16(const float* v, float s, float r) {
 // doubles).  The caller guarantees red is no longer being read (a barrier at
 // the top of the row, or a copy of red per row parity), so one barrier
 // suffices.
+// Sum over the wave in every lane, the additions of xor steps 32, 16, 8, 4, 2,
+// 1: lane swaps across halves and rows of 16, then rotations inside the rows
+// (after step 8 a rotation by 4 reaches the same pair sum as xor 4, and so
+// on).  As LDS shuffles the twelve steps of a row's two sums were ~0.4 us of
+// its latency.
+IC_DEV double wave_sum_f64(double v) {
+  auto dbl = [](uint32_t lo, uint32_t hi) { return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo)); };
+  auto lo_of = [](double d) { return (uint32_t)__double_as_longlong(d); };
+  auto hi_of = [](double d) { return (uint32_t)((uint64_t)__double_as_longlong(d) >> 32); };
+  {
+    const auto l = __builtin_amdgcn_permlane32_swap(lo_of(v), lo_of(v), false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi_of(v), hi_of(v), false, false);
+    v = dbl(l[0], h[0]) + dbl(l[1], h[1]);
+  }
+  {
+    const auto l = __builtin_amdgcn_permlane16_swap(lo_of(v), lo_of(v), false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi_of(v), hi_of(v), false, false);
+    v = dbl(l[0], h[0]) + dbl(l[1], h[1]);
+  }
+#define IC_ROR(N) \
+  v += dbl((uint32_t)__builtin_amdgcn_mov_dpp((int)lo_of(v), 0x120 + N, 0xf, 0xf, false), \
+           (uint32_t)__builtin_amdgcn_mov_dpp((int)hi_of(v), 0x120 + N, 0xf, 0xf, false))
+  IC_ROR(8);
+  IC_ROR(4);
+  IC_ROR(2);
+  IC_ROR(1);
+#undef IC_ROR
+  return v;
+}
+
 template <int TH>
 IC_DEV void block_sum2_f64(double& a, double& b, double* red) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    a += __shfl_xor(a, o, 64);
-    b += __shfl_xor(b, o, 64);
-  }
+  a = wave_sum_f64(a);
+  b = wave_sum_f64(b);
   if ((threadIdx.x & 63) == 0) {
     red[2 * (threadIdx.x >> 6)] = a;
     red[2 * (threadIdx.x >> 6) + 1] = b;
@@ -79,57 +106,18 @@ IC_DEV void block_sum2_f64(double& a, double& b, double* red) {
   }
 }
 
-// TH threads per workgroup (256; 192 = three waves for rows of up to 3072 or
-// 6144 values, 320 = five waves for rows of 4097..5120 values and 448 = seven
-// for 12289..14336, all with R <= 1024, whose Hadamard exchange stays inside a
-// wave): a tile is TH * 16 positions.  For R = 1024 a wave's 64 x 16 positions are exactly one block,
-// so its last digit is exchanged through the wave's own slice of the LDS
-// buffer, without a workgroup barrier.
-//
-// NORM (IC_NORM_LAYER / IC_NORM_RMS, ic_norm_rotate_quantize): before the
-// prep, the row is normalised and rounded once to DT,
-//   y = RN_dt(f32(f32(f32(x - mean) * rstd) * nw[k]) + nb[k])     (LayerNorm)
-//   y = RN_dt(f32(f32(x * rstd) * nw[k]) + nb[k])                  (RMSNorm)
-// (nw / nb optional), mean = RN32(S1 / K_in) and rstd = RN32(1 / sqrt(V / K_in
-// + eps)) from fp64 sums over the row the registers already hold: one pass,
-// V = S2 - S1^2 / K_in with S1 = sum x, S2 = sum x^2 (the sums of 16-bit
-// values are exact in fp64 for any realistic row).  The prep
-// then treats y as its input: the same arithmetic as the chain normalise ->
-// activation tensor -> rotate_quantize, without the tensor.
-// (the 768-thread workgroup, and the two-tile 448 / 512-thread ones with a
-// row buffer, leave LDS for one workgroup per CU, which their launch bounds
-// say)
-template <int DT, int LOG4R, int NT, int VAR, int TH>
-constexpr int rq_fast_min_wgs() {
-  const bool wave_local = VAR == kRqPlain && LOG4R >= 3 && LOG4R <= 5 && NT <= 2;
-  if (TH >= 768 || (TH >= 448 && NT >= 2 && !wave_local)) return 1;
-  return (NT <= 3 || VAR == kRqPlain) ? 2 : 1;
-}
-//
-// QUANT false (ic_prepare_activation): the prepared row itself leaves, in DT,
-// gathered from the same row buffer; no abs-max and no codes.  One workgroup
-// per row and a re-read of factors and perm for each row (rotate_quant_kernel,
-// which still serves the forms this kernel does not take) took 61.9 us for
-// 4608 x 3072 at R = 256 with both, this kernel 27.9 us.
-template <int DT, int LOG4R, int NT, int VAR, int TH, int NORM = 0, bool QUANT = true>
-__global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) void rq_fast_kernel(
-    const u16* __restrict__ x, int64_t ldx, int M, int K_in, int K_r,
-    const float* __restrict__ sr_rcp, const float* __restrict__ sr_f, int K_w,
-    const int32_t* __restrict__ perm, int8_t* __restrict__ q_out, int64_t ldq,
-    float* __restrict__ s_out, const float* __restrict__ nw, const float* __restrict__ nb, float eps,
-    u16* __restrict__ y_out, int64_t ldy) {
-  static_assert(QUANT || NORM == 0, "the normalising kernels quantize");
-  constexpr int RC = LOG4R <= 2 ? 0 : (LOG4R <= 4 ? 1 : (LOG4R == 5 ? 3 : 2));
-  constexpr bool XCH = LOG4R >= 3;
-  constexpr int kTile = TH * 16;  // positions per tile
-  static_assert(TH == 256 || (TH % 64 == 0 && LOG4R <= 5), "cross-wave rotation needs four waves");
+// The LDS of one instantiation and what follows from it.
+template <int DT, int LOG4R, int NT, int VAR, int TH, int NORM>
+struct RqLds {
+  static constexpr bool XCH = LOG4R >= 3;
+  static constexpr int kTile = TH * 16;  // positions per tile
   // WLR: rows without a perm whose rotation stays inside each wave's 1024
   // positions (R = 64..1024 with the DMA-staged slices, at most two tiles)
   // keep their rounded values in the upper half of the wave's own exchange
   // slice instead of a row buffer: the quantization then reads only what
   // its own wave wrote, and the workgroup needs no row-sized buffer (the
   // Wan FFN-down rows fit two workgroups per CU instead of one).
-  constexpr bool WLR = VAR == kRqPlain && XCH && LOG4R <= 5 && NT <= 2;
+  static constexpr bool WLR = VAR == kRqPlain && XCH && LOG4R <= 5 && NT <= 2;
   // DBR: the row buffer and the reduction slots alternate between two copies
   // by row parity, so no barrier is needed at the top of a row: a wave that
   // writes row r + 2's copy has passed row r + 1's abs-max barrier, which no
@@ -152,24 +140,70 @@ __global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) vo
   // (3 - (a ^ 2) = (3 - a) ^ 2), so the butterflies run unchanged and only
   // the row-buffer stores (and the test of pad positions) use the logical
   // index j ^ 8.
-  constexpr int kRowLen = WLR ? 8 : rowbuf_len<NT, kTile>();
-  constexpr int kWgCap = 1024 / TH;  // ~16 waves per CU at these kernels' register counts
+  static constexpr int kRowLen = WLR ? 8 : rowbuf_len<NT, kTile>();
+  static constexpr int kWgCap = 1024 / TH;  // ~16 waves per CU at these kernels' register counts
   // the reduction slots (NB copies) and 32 bytes of alignment
-  constexpr int kSlots1 = (TH / 64) * 4 + (NORM != 0 ? 2 * (TH / 64) : 1) * 8 +
+  static constexpr int kSlots1 = (TH / 64) * 4 + (NORM != 0 ? 2 * (TH / 64) : 1) * 8 +
                           (DT == IC_DTYPE_BF16 && LOG4R == 6 ? 2 * (TH / 64) : 1) * 4 + 32;
-  constexpr int kSlots2 = kSlots1 + (TH / 64) * 4 + (NORM != 0 ? 2 * (TH / 64) : 1) * 8;
+  static constexpr int kSlots2 = kSlots1 + (TH / 64) * 4 + (NORM != 0 ? 2 * (TH / 64) : 1) * 8;
   // workgroups per CU with one or two row buffers and an exchange buffer of
   // XB bytes (LDS is allocated in 512-byte granules)
-  constexpr auto occ = [](int xb, int nbuf) {
+  static constexpr int occ(int xb, int nbuf) {
     const int lds = (xb + 2 * nbuf * kRowLen + (nbuf == 1 ? kSlots1 : kSlots2) + 511) / 512 * 512;
     return 163840 / lds < kWgCap ? 163840 / lds : kWgCap;
-  };
-  constexpr auto dbr_fits = [occ](int xb) { return occ(xb, 2) >= 1 && occ(xb, 2) >= occ(xb, 1); };
-  constexpr int kXbPad = XCH ? 8 * xbuf_doubles<kTile>() : 16;
-  constexpr int kXbTight = XCH ? 8 * tslot_doubles<kTile>() : 16;
-  constexpr bool XROT = XCH && (LOG4R == 3 || LOG4R == 4) && !WLR && kWgCap >= 2 && !dbr_fits(kXbPad) &&
-                        dbr_fits(kXbTight);
-  constexpr bool DBR = LOG4R <= 5 && (WLR || dbr_fits(XROT ? kXbTight : kXbPad));
+  }
+  static constexpr bool dbr_fits(int xb) { return occ(xb, 2) >= 1 && occ(xb, 2) >= occ(xb, 1); }
+  static constexpr int kXbPad = XCH ? 8 * xbuf_doubles<kTile>() : 16;
+  static constexpr int kXbTight = XCH ? 8 * tslot_doubles<kTile>() : 16;
+  static constexpr bool XROT = XCH && (LOG4R == 3 || LOG4R == 4) && !WLR && kWgCap >= 2 &&
+                        ((!dbr_fits(kXbPad) && dbr_fits(kXbTight)) || occ(kXbTight, 1) > occ(kXbPad, 1));
+  static constexpr bool DBR = LOG4R <= 5 && (WLR || dbr_fits(XROT ? kXbTight : kXbPad));
+  // Waves per SIMD that the LDS admits, which the registers then have to (the
+  // compiler otherwise took up to 184 and left one workgroup of two or three).
+  // At most three (168 registers; four spill), four where two seven-wave
+  // workgroups need them.
+  static constexpr int kWgs = occ(XROT ? kXbTight : kXbPad, DBR ? 2 : 1);
+  static constexpr int kWaves = (kWgs * (TH / 64) + 3) / 4;
+  static constexpr int kMinWaves = kWaves < 3 ? (kWaves < 1 ? 1 : kWaves) : (TH == 448 && NT == 1 && NORM == 0 ? kWaves : 3);
+};
+
+// TH threads per workgroup: a tile is TH * 16 positions, and for R <= 1024 any
+// number of waves will do, since the Hadamard exchange stays inside a wave
+// (launch_fast_nt has the widths).  For R = 1024 a wave's 64 x 16 positions are
+// exactly one block, so its last digit is exchanged through the wave's own
+// slice of the LDS buffer, without a workgroup barrier.
+//
+// NORM (IC_NORM_LAYER / IC_NORM_RMS, ic_norm_rotate_quantize): before the
+// prep, the row is normalised and rounded once to DT,
+//   y = RN_dt(f32(f32(f32(x - mean) * rstd) * nw[k]) + nb[k])     (LayerNorm)
+//   y = RN_dt(f32(f32(x * rstd) * nw[k]) + nb[k])                  (RMSNorm)
+// (nw / nb optional), mean = RN32(S1 / K_in) and rstd = RN32(1 / sqrt(V / K_in
+// + eps)) from fp64 sums over the row the registers already hold: one pass,
+// V = S2 - S1^2 / K_in with S1 = sum x, S2 = sum x^2 (the sums of 16-bit
+// values are exact in fp64 for any realistic row).  The prep
+// then treats y as its input: the same arithmetic as the chain normalise ->
+// activation tensor -> rotate_quantize, without the tensor.
+//
+// QUANT false (ic_prepare_activation): the prepared row itself leaves, in DT,
+// gathered from the same row buffer; no abs-max and no codes.  One workgroup
+// per row and a re-read of factors and perm for each row (rotate_quant_kernel,
+// which still serves the forms this kernel does not take) took 61.9 us for
+// 4608 x 3072 at R = 256 with both, this kernel 27.9 us.
+template <int DT, int LOG4R, int NT, int VAR, int TH, int NORM = 0, bool QUANT = true>
+__global__ __launch_bounds__(TH, (RqLds<DT, LOG4R, NT, VAR, TH, NORM>::kMinWaves)) void rq_fast_kernel(
+    const u16* __restrict__ x, int64_t ldx, int M, int K_in, int K_r,
+    const float* __restrict__ sr_rcp, const float* __restrict__ sr_f, int K_w,
+    const int32_t* __restrict__ perm, int8_t* __restrict__ q_out, int64_t ldq,
+    float* __restrict__ s_out, const float* __restrict__ nw, const float* __restrict__ nb, float eps,
+    u16* __restrict__ y_out, int64_t ldy) {
+  static_assert(QUANT || NORM == 0, "the normalising kernels quantize");
+  constexpr int RC = LOG4R <= 2 ? 0 : (LOG4R <= 4 ? 1 : (LOG4R == 5 ? 3 : 2));
+  constexpr bool XCH = LOG4R >= 3;
+  constexpr int kTile = TH * 16;  // positions per tile
+  using L = RqLds<DT, LOG4R, NT, VAR, TH, NORM>;
+  constexpr bool WLR = L::WLR, XROT = L::XROT, DBR = L::DBR;
+  constexpr int kRowLen = L::kRowLen;
+  static_assert(TH == 256 || (TH % 64 == 0 && LOG4R <= 5), "cross-wave rotation needs four waves");
   __shared__ double xbuf[XCH ? (XROT ? tslot_doubles<kTile>() : xbuf_doubles<kTile>()) : 2];
   auto xs = [](int p) { return XROT ? tslot(p) : xslot(p); };
   constexpr int NB = DBR ? 2 : 1;
@@ -364,9 +398,9 @@ __global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) vo
         float xs[16];
         unpack8<DT>(xa, xs);
         unpack8<DT>(xb, xs + 8);
-        float xn[NORM != 0 ? 16 : 1];  // normalised run, the divide's input
-        if constexpr (NORM != 0) {
-          if (p0 < K_in) {  // pad runs stay zero
+        // normalised run, the divide's input (the exact path below forms it again)
+        auto norm_run = [&](float* xs) {
+          if (NORM != 0 && p0 < K_in) {  // pad runs stay zero
             float w[16], b[16];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -383,9 +417,8 @@ __global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) vo
               xs[j] = round_to_dt<DT>(y);
             }
           }
-#pragma unroll
-          for (int j = 0; j < 16; ++j) xn[j] = xs[j];
-        }
+        };
+        norm_run(xs);
         // bf16: the run's |x| extremes for the flush rule, formed with the
         // divide's own range test where there is one
         Bf16RunStats fst{0u, 0.0f};
@@ -430,13 +463,9 @@ __global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) vo
             fst_ok = false;  // the exact path below replaces the run
             if (p0 < K_in) {
               float xo[16];
-              if constexpr (NORM != 0) {
-#pragma unroll
-                for (int j = 0; j < 16; ++j) xo[j] = xn[j];
-              } else {
-                unpack8<DT>(xa, xo);
-                unpack8<DT>(xb, xo + 8);
-              }
+              unpack8<DT>(xa, xo);
+              unpack8<DT>(xb, xo + 8);
+              norm_run(xo);
 #pragma unroll
               for (int j = 0; j < 16; ++j) {
                 xs[j] = div_round_dt<DT>(xo[j], rc[PLAIN ? 0 : c][j], sr_f, p0 + j);
@@ -518,27 +547,32 @@ __global__ __launch_bounds__(TH, (rq_fast_min_wgs<DT, LOG4R, NT, VAR, TH>())) vo
         }
       }
       if (c + 1 == NT || base + kTile >= K_w) __builtin_amdgcn_s_setprio(1);
-      // ---- round once to DT: RN32 first; exact round-to-odd for the rare runs
-      // holding a DT rounding boundary, a tiny value or a zero, and for the
-      // runs of a tile that reaches into the pad to K_w (zeroed there)
+      // ---- round once to DT: round-to-odd to 21 bits (rto_hi), exact for every
+      // value in f32's normal range; bf16 runs holding a zero or a value below it
+      // take the 24-bit form.  A tile that reaches into the pad to K_w zeroes it.
+      // (Before, RN32 with a second look at the runs that held a rounding
+      // boundary: sums of 11-bit values lie on one often enough that nearly every
+      // wave ran its 136 instructions, a quarter of the row's.  C3 PREPA.)
       float z[16];
       float zmin = __builtin_huge_valf(), zmax = 0.0f;
-      uint32_t bmin = 0xffffffffu;  // zero iff some z[j] is a DT boundary
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        z[j] = (float)v[j];
-        zmin = __builtin_fminf(zmin, __builtin_fabsf(z[j]));
+        z[j] = rto_hi(v[j]);
+        if constexpr (DT == IC_DTYPE_BF16) zmin = __builtin_fminf(zmin, __builtin_fabsf(z[j]));
         zmax = __builtin_fmaxf(zmax, __builtin_fabsf(z[j]));
-        const uint32_t key = rn32_boundary_key<DT>(z[j]);
-        bmin = bmin < key ? bmin : key;
       }
-      if (__builtin_expect(bmin == 0u || !(zmin >= dt_min_normal<DT>()) || base + kTile > K_r, 0)) {
+      if (DT == IC_DTYPE_BF16 && __builtin_expect(!(zmin >= dt_min_normal<DT>()), 0)) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) z[j] = rto24(v[j]);
+      }
+      int kr = K_r;
+      asm volatile("" : "+s"(kr));  // else the compiler makes two copies of the row loop
+      if (base + kTile > kr) {  // uniform
         zmax = 0.0f;
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          z[j] = rto24(v[j]);
           const int jl = XROT ? (j ^ (8 * ((t >> 5) & 1))) : j;  // logical index of register j
-          if (base + kTile > K_r && base + tile_pos<(LOG4R == 0 ? 0 : RC)>(t, jl) >= K_r) z[j] = 0.0f;
+          if (base + tile_pos<(LOG4R == 0 ? 0 : RC)>(t, jl) >= K_r) z[j] = 0.0f;
           zmax = __builtin_fmaxf(zmax, __builtin_fabsf(z[j]));
         }
       }
@@ -803,34 +837,52 @@ hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
   return hipGetLastError();
 }
 
+//
+// Workgroup widths.  R <= 1024: one wave per 1024 positions and one tile, so that
+// no wave is idle and a row's latency is one tile's; 256-thread workgroups with
+// 1 to 3 idle waves before.  us before -> now (R = 256, factors and perm):
+//   20000 x 1024 97 -> 25, 10000 x 2048 51 -> 24, 4608 x 5120 48 -> 46,
+//   4608 x 7168 52 -> 40, 64 x 6144 7.2 -> 5.2; RMSNorm first, 24409 x 2048 142 -> 70
+// Two tiles of three or four waves instead where one wide tile leaves a single
+// workgroup per CU or too few registers: eight waves (4608 x 8192 48.6 against
+// 52.9), seven and up to six with a norm (LayerNorm, 4608 x 5120: 46.8 against
+// 79 on five waves), and five or six unrotated (no LDS exchange to shorten).
 template <int DT, int LOG4R, int VAR, int NORM = 0, bool QUANT = true>
 hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
-  if constexpr (LOG4R == 5) {
-    // five one-block waves cover 4097..5120 values in one tile (Wan's 5120
-    // would otherwise take two 4096-tiles, 37.5 % of them padding)
-    if (a.K_w > kTile && a.K_w <= 320 * 16) return launch_fast_t<DT, LOG4R, 1, VAR, 320, NORM, QUANT>(a, st);
-    // seven one-block waves, two tiles: 12289..14336 values (Wan's FFN-down
-    // 14336 instead of four 4096-tiles; ~99 KB of LDS, one workgroup per CU)
-    if (a.K_w > 3 * kTile && a.K_w <= 2 * 448 * 16) return launch_fast_t<DT, LOG4R, 2, VAR, 448, NORM, QUANT>(a, st);
-  }
-  if constexpr (LOG4R >= 3 && LOG4R <= 5) {
-    // one tile of twelve waves for 8193..12288 values (Flux's 12288): the
-    // per-thread constants of one tile instead of three
-    if (a.K_w > 2 * kTile && a.K_w <= 768 * 16) return launch_fast_t<DT, LOG4R, 1, VAR, 768, NORM, QUANT>(a, st);
-    // two tiles of eight waves for 12289..16384 (Flux's single-block 15360)
-    if (a.K_w > 3 * kTile) return launch_fast_t<DT, LOG4R, 2, VAR, 512, NORM, QUANT>(a, st);
-  }
+#define IC_RQ(NT, TH) return launch_fast_t<DT, LOG4R, NT, VAR, TH, NORM, QUANT>(a, st)
   if constexpr (LOG4R <= 5) {
-    // three-wave workgroups where their tile fits the row more tightly
-    // (3072: one full tile instead of 3/4 of one; 4097..6144: two)
-    constexpr int T3 = 192 * 16;
-    if (a.K_w <= T3 && a.K_w > kTile / 2) return launch_fast_t<DT, LOG4R, 1, VAR, 192, NORM, QUANT>(a, st);
-    if (a.K_w > kTile && a.K_w <= 2 * T3) return launch_fast_t<DT, LOG4R, 2, VAR, 192, NORM, QUANT>(a, st);
+    switch ((a.K_w + 1023) / 1024) {
+      case 1: IC_RQ(1, 64);
+      case 2: IC_RQ(1, 128);
+      case 3: IC_RQ(1, 192);
+      case 4: IC_RQ(1, 256);
+      case 5:
+        if constexpr (NORM == 0 && LOG4R >= 3) IC_RQ(1, 320);
+        IC_RQ(2, 192);
+      case 6:
+        if constexpr (NORM == 0 && LOG4R >= 3) IC_RQ(1, 384);
+        IC_RQ(2, 192);
+      case 7:
+        if constexpr (NORM == 0 && RqLds<DT, LOG4R, 1, VAR, 448, NORM>::kWgs >= 2) IC_RQ(1, 448);
+        IC_RQ(2, 256);
+      case 8: IC_RQ(2, 256);
+      case 9:
+      case 10:
+      case 11:
+      case 12: IC_RQ(1, 768);
+      case 13:
+      case 14:
+        if constexpr (LOG4R == 5) IC_RQ(2, 448);
+        break;
+    }
+    IC_RQ(2, 512);
+  } else {
+    if (a.K_w <= kTile) IC_RQ(1, kThreads);
+    if (a.K_w <= 2 * kTile) IC_RQ(2, kThreads);
+    if (a.K_w <= 3 * kTile) IC_RQ(3, kThreads);
+    IC_RQ(4, kThreads);
   }
-  if (a.K_w <= kTile) return launch_fast_t<DT, LOG4R, 1, VAR, kThreads, NORM, QUANT>(a, st);
-  if (a.K_w <= 2 * kTile) return launch_fast_t<DT, LOG4R, 2, VAR, kThreads, NORM, QUANT>(a, st);
-  if (a.K_w <= 3 * kTile) return launch_fast_t<DT, LOG4R, 3, VAR, kThreads, NORM, QUANT>(a, st);
-  return launch_fast_t<DT, LOG4R, 4, VAR, kThreads, NORM, QUANT>(a, st);
+#undef IC_RQ
 }
 
 // VAR must match the arguments (the per-dtype dispatcher routes on them).
