@@ -38,6 +38,7 @@
 #include "gemm_i8_big.h"
 #include "gemm_mid_plan.h"
 #include "rq_common.h"
+#include "splitk_reduce.h"
 
 // GEMM launches with the activation / residual epilogue compiled in
 // (gemm_i8_epi.hip).
@@ -813,6 +814,14 @@ hipError_t launch_mfma(const GemmArgs& g, hipStream_t st) {
       hipError_t e = launch_kernel<TL, OUT_DT, false, true, EPI>(g, S, st);
       if (e != hipSuccess) return e;
       const int64_t MN = (int64_t)g.M * g.N;
+      if constexpr (OUT_DT != IC_DTYPE_F32) {
+        if (g.N % 4 == 0 && g.ldc % 4 == 0 && (((uintptr_t)g.C) & 7) == 0 && (((uintptr_t)g.ws) & 15) == 0) {
+          constexpr int KIND = TL::GS != 0 ? 2 : (TL::INT4 ? 1 : 0);
+          splitk_reduce4_kernel<KIND, OUT_DT><<<dim3((unsigned)((MN / 4 + 255) / 256)), dim3(256), 0, st>>>(
+              (const int32_t*)g.ws, S, g.s_a, g.s_w, g.bias, g.bias_dt, g.C, g.ldc, g.M, g.N, g.epi);
+          return hipGetLastError();
+        }
+      }
       splitk_reduce_kernel<TL::INT4, TL::GS, OUT_DT><<<dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, st>>>(
           (const int32_t*)g.ws, S, g.s_a, g.s_w, g.bias, g.bias_dt, g.C, g.ldc, g.M, g.N, g.epi);
       return hipGetLastError();

@@ -18,12 +18,13 @@
 //
 // PART (split-K): workgroup (x, y) computes K slice y of gridDim.y and writes
 // 4-byte partials (int32 sums, or the fp32 fold) to
-// ws[(y * M + m) * N + n]; mid_reduce_kernel adds them in slice order.
+// ws[(y * M + m) * N + n]; splitk_reduce4_kernel adds them in slice order.
 #pragma once
 #include <type_traits>
 
 #include "gemm_i8_big.h"
 #include "gemm_mid_plan.h"
+#include "splitk_reduce.h"
 
 namespace {
 namespace mid {
@@ -367,51 +368,6 @@ __global__ __launch_bounds__(mid::kMT, 2) void gemm_mid_kernel(
   }
 }
 
-// Adds the K-slice partials in slice order and finishes the outputs as the
-// unsplit epilogue does, four columns per thread (N a multiple of 4; staged
-// 16-bit outputs).  KIND 0: int32 sums and per-row scales (1: of 16 * q
-// weights), 2: fp32 folds of groups, 3: fp32 sums (W4A16).
-template <int KIND, int OUT_DT>
-__global__ __launch_bounds__(256) void mid_reduce_kernel(
-    const int32_t* __restrict__ ws, int S, const float* __restrict__ s_a, const float* __restrict__ s_w,
-    const void* __restrict__ bias, int bias_dt, void* __restrict__ C, int64_t ldc, int M, int N, ic_epi epi) {
-  const int64_t MN = (int64_t)M * N;
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i >= MN) return;
-  const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
-  float v[4];
-  if constexpr (KIND < 2) {
-    v4i t = *(const v4i*)(ws + i);
-    for (int s = 1; s < S; ++s) t = t + *(const v4i*)(ws + s * MN + i);
-    const float sa = s_a[m];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      float a = (float)t[k];
-      if constexpr (KIND == 1) a *= 0.0625f;
-      v[k] = a * (sa * s_w[n + k]);
-    }
-  } else {
-    v4f t = *(const v4f*)((const float*)ws + i);
-    for (int s = 1; s < S; ++s) {
-      const v4f u = *(const v4f*)((const float*)ws + s * MN + i);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) t[k] = t[k] + u[k];
-    }
-    const float sa = KIND == 2 ? s_a[m] : 1.0f;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = KIND == 2 ? t[k] * sa : t[k];
-  }
-  u16 h[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (bias != nullptr) v[k] = v[k] + ld_any_f32(bias, bias_dt, n + k);
-    v[k] = epi_apply(v[k], epi, m, n + k);
-    h[k] = OUT_DT == IC_DTYPE_F16 ? f32_to_f16(v[k]) : f32_to_bf16(v[k]);
-  }
-  *(v2u*)((u16*)C + (int64_t)m * ldc + n) =
-      v2u{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
-}
-
 // Ring depths that let two (packed 32- and 64-row tiles: three or four)
 // workgroups share a CU's 160 KB of LDS.
 template <int T, int MODE>
@@ -447,7 +403,7 @@ hipError_t launch_mid_t(const ic_gemm::GemmArgs& g, int S, hipStream_t st) {
   if (hipError_t e = launch_mid_k<T, MODE, PDT, false, KIL, true>(g, S, st)) return e;
   constexpr int KIND = MODE == big::ROW8 ? 0 : (MODE == big::ROW4 ? 1 : (MODE == big::W16 ? 3 : 2));
   const int64_t q = (int64_t)g.M * g.N / 4;
-  mid_reduce_kernel<KIND, OUT_DT><<<dim3((unsigned)((q + 255) / 256)), dim3(256), 0, st>>>(
+  splitk_reduce4_kernel<KIND, OUT_DT><<<dim3((unsigned)((q + 255) / 256)), dim3(256), 0, st>>>(
       (const int32_t*)g.ws, S, g.s_a, g.s_w, g.bias, g.bias_dt, g.C, g.ldc, g.M, g.N, g.epi);
   return hipGetLastError();
 }
