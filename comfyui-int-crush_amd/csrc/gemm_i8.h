@@ -934,11 +934,14 @@ double tile_us(const GemmArgs& g, bool grouped, const TileShape& t, int S) {
 // launch chosen otherwise, in S0 slices).  Grouped launches keep its slices:
 // a slice boundary moves the order of the fp32 fold, and the outputs of a
 // shape do not depend on the kernel (nor on the output type, whose f32 form
-// only the other tiles write).  Per-row sums are exact in any slices.
+// only the other tiles write).  Per-row sums are exact in any slices.  The
+// reduction loads 16 bytes of a workspace: one that is not aligned to them
+// leaves a launch unsplit, or on the other tiles.
 bool mid_pick(const GemmArgs& g, int mode, bool grouped, int S0, double base, MidPlan& p) {
-  if (!mid_rounds_ok(g.M, g.N)) return false;
+  const bool ws_ok = g.ws != nullptr && (((uintptr_t)g.ws) & 15) == 0;
+  if (!mid_rounds_ok(g.M, g.N) || (grouped && S0 > 1 && !ws_ok)) return false;
   const int64_t mn4 = (int64_t)g.M * g.N * 4;
-  const int64_t fit = g.ws != nullptr ? g.ws_bytes / mn4 : 0;
+  const int64_t fit = ws_ok ? g.ws_bytes / mn4 : 0;
   const int most = fit > 16 ? 16 : (fit < 1 ? 1 : (int)fit);
   p = grouped ? mid_plan(mode, g.M, g.N, g.K / kBK, S0, S0) : mid_plan(mode, g.M, g.N, g.K / kBK, 1, most);
   return p.us < base;

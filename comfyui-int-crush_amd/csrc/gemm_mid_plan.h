@@ -11,11 +11,12 @@
 //          slices 16.5
 //   g64    146 x 1312 x 8448: 32 x 64 29.7, 64 x 64 43.1; 256 x 192 125.5
 //   W4A16  63 x 3256 x 3712: 64 x 64 33.8, in four slices 16.5; 128 x 256 68.9
-// The large tiles stay ahead once they fill the CUs, and past two rounds of
-// them the small ones are not looked at (mid_rounds_ok): the estimates leave
-// out the epilogues' memory time, which weighs on short K (W8A8 19053 x 10992 x
-// 1152 with GELU and a residual: 608 us on 320 x 192 tiles, 624 us on 128 x 128) (W8A8 1111 x 9216 x 3072:
-// 35.6 against 43.8 us; g128 1357 x 7688 x 2560: 40.7 against 49.4).
+// The large tiles stay ahead once they fill the CUs (W8A8 1111 x 9216 x 3072:
+// 35.6 against 43.8 us; g128 1357 x 7688 x 2560: 40.7 against 49.4), and past
+// two rounds of them the small ones are not looked at (mid_rounds_ok): the
+// estimates leave out the epilogues' memory time, which weighs on short K
+// (W8A8 19053 x 10992 x 1152 with GELU and a residual: 608 us on 320 x 192
+// tiles, 624 us on 128 x 128).
 #pragma once
 #include "gemm_common.h"
 

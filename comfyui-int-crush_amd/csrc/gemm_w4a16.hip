@@ -5,7 +5,9 @@
 // weight w[n,k] = RN_dt(q[n,k] * RN_dt(s[n, k/gs])) is never written to HBM.
 // Shapes with M > 128, groups of whole 64-column blocks and an aligned 16-bit
 // output run gemm_i8_big_kernel's W4A16 mode (weights dequantized in registers,
-// v_mfma_f32_16x16x32); the kernel below covers the rest: the dequantized tile
+// v_mfma_f32_16x16x32), or its arithmetic on small tiles (gemm_mid.h) where
+// few tiles would leave CUs idle, M <= 128 included; the kernel below covers
+// the rest: the dequantized tile
 // is produced in LDS and consumed by v_mfma_f32_32x32x16_{f16,bf16}.  For
 // fp16 this is bit-identical to the reference unpack (an fp16 product of two
 // fp16 values); the reference rejects bf16 here and its PyTorch fallback
@@ -402,8 +404,9 @@ MidPlan w16_plan(int64_t M, int64_t N, int64_t K, int max_s) {
   return p;
 }
 constexpr int kW16MaxSplits = 16;
+// the reduction's loads take a workspace aligned to 16 bytes
 int w16_max_splits(int64_t M, int64_t N, const void* ws, int64_t ws_bytes) {
-  const int64_t fit = ws != nullptr ? ws_bytes / (M * N * 4) : 0;
+  const int64_t fit = ws != nullptr && ((uintptr_t)ws & 15) == 0 ? ws_bytes / (M * N * 4) : 0;
   return fit > kW16MaxSplits ? kW16MaxSplits : (fit < 1 ? 1 : (int)fit);
 }
 

@@ -837,7 +837,6 @@ hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-//
 // Workgroup widths.  R <= 1024: one wave per 1024 positions and one tile, so that
 // no wave is idle and a row's latency is one tile's; 256-thread workgroups with
 // 1 to 3 idle waves before.  us before -> now (R = 256, factors and perm):

@@ -5,11 +5,12 @@
 namespace {
 
 // Adds the K-slice partials in slice order and finishes the outputs as the
-// unsplit epilogue does, four columns per thread (N and ldc multiples of 4, C
-// 8-byte and ws 16-byte aligned): 16-byte loads of the partials, where one column
-// per thread left the two kernels of 512 x 3072 x 12288 in two slices with a
-// residual at 45.7 us against 44.4.  KIND 0: int32 sums and per-row scales (1: of 16 * q
-// weights), 2: fp32 folds of groups, 3: fp32 sums (W4A16).
+// unsplit epilogue does.  Bound by the partials' reads: four columns per
+// thread (N and ldc multiples of 4, C 8-byte and ws 16-byte aligned) make them
+// 16-byte loads.  512 x 3072 x 12288 W4A8 in two slices with a residual: this
+// kernel 7.4 -> 6.2 us, both kernels 45.7 -> 44.4.  KIND 0: int32 sums and
+// per-row scales (1: of 16 * q weights), 2: fp32 folds of groups, 3: fp32 sums
+// (W4A16).
 template <int KIND, int OUT_DT>
 __global__ __launch_bounds__(256) void splitk_reduce4_kernel(
     const int32_t* __restrict__ ws, int S, const float* __restrict__ s_a, const float* __restrict__ s_w,

@@ -176,7 +176,8 @@ int ic_gemm_w4a8(const int8_t* xq, int64_t M, int64_t K, int64_t ldx, const uint
  * scale outputs are bit-identical to the unsplit GEMM; grouped outputs differ
  * only in the order of the fp32 additions.  ic_gemm_splitk_bytes returns the
  * most workspace a launch of that shape uses (0: no split; then workspace may
- * be null); a smaller workspace than that runs on fewer slices or unsplit.
+ * be null); a smaller workspace than that runs on fewer slices or unsplit, as
+ * one not aligned to 16 bytes may.
  * Launches with 16-bit, 16-byte aligned outputs may take small tiles instead,
  * in fewer slices or none.  The library itself
  * never allocates.
@@ -343,8 +344,9 @@ int ic_gemm_w4a16_staged(const void* x, int dtype, int64_t M, int64_t K, int64_t
  * output tiles leave most CUs idle: K slices run in parallel, their fp32 sums
  * go to the caller's workspace and a second kernel adds them in slice order.
  * ic_gemm_w4a16_splitk_bytes is the workspace such a launch uses (0: no
- * split); with less, or none, it runs on fewer slices or unsplit, as the
- * entry points without a workspace do.  No reference counterpart.
+ * split); with less it runs on fewer slices, with none, or one not aligned to
+ * 16 bytes, unsplit, as the entry points without a workspace do.  No reference
+ * counterpart.
  */
 int64_t ic_gemm_w4a16_splitk_bytes(int64_t M, int64_t N, int64_t K, int64_t num_groups);
 int ic_gemm_w4a16_ws(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_packed,

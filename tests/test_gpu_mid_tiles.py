@@ -92,3 +92,36 @@ def test_w4a16_small_tiles(rt, dev, dtype, group):
         rt._call("ic_gemm_w4a16", rt._ptr(x), rt._dt(dtype, ""), M, K, K, rt._ptr(w), N, K // 2, rt._ptr(s), K // gs,
                  rt._ptr(b), rt._dt(dtype, ""), rt._ptr(o2), N, rt._stream(x))
         assert bool(((o2.double() - ref).abs() <= bound).all()), (M, N, K)
+
+
+def test_workspace_not_aligned_to_16_bytes(rt, dev):
+    """The split reductions load 16 bytes of partials at a time; any workspace
+    that was accepted before still is, and gives the same results."""
+    M, N, K = 40, 256, 8192
+    g = torch.Generator().manual_seed(5)
+    st, bf = rt._stream(torch.empty(1, device=dev)), rt._dt(torch.bfloat16, "")
+    x, s_a = _codes(M, K, g, dev), (torch.rand(M, generator=g) * 1e-2).to(dev)
+    xf = torch.randn(M, K, generator=g).to(torch.bfloat16).to(dev)
+    w8 = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).to(dev)
+    w4 = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8).to(dev)
+    s_w = (torch.rand(N, K // 128, generator=g) * 1e-2).to(dev)
+    s_row = s_w[:, 0].contiguous()
+    size = max(rt.lib().ic_gemm_splitk_bytes(M, N, K, G, i4) for G, i4 in ((1, 0), (K // 128, 1)))
+    size = max(size, rt.lib().ic_gemm_w4a16_splitk_bytes(M, N, K, K // 128))
+    assert size > 0
+    buf = torch.empty(size + 64, dtype=torch.uint8, device=dev)
+    p = rt._ptr
+
+    def run(entry, *args, ws):
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+        tail = (p(buf[ws:]), size) if ws is not None else ()
+        rt._call(entry, *args[:-1], *args[-1], p(out), *((bf,) if "w4a16" not in entry else ()), N, *tail, st)
+        return out
+
+    a8 = (p(x), M, K, K, p(w8), N, K, p(s_a), p(s_row), (None, 0))
+    a4 = (p(x), M, K, K, p(w4), N, K // 2, p(s_w), K // 128, p(s_a), (None, 0))
+    a16 = (p(xf), bf, M, K, K, p(w4), N, K // 2, p(s_w), K // 128, (None, 0))
+    for ws in (4, 8):
+        assert torch.equal(run("ic_gemm_w8a8_ws", *a8, ws=ws), run("ic_gemm_w8a8_ws", *a8, ws=0))
+        assert torch.equal(run("ic_gemm_w4a8_ws", *a4, ws=ws), run("ic_gemm_w4a8_ws", *a4, ws=0))
+        assert torch.equal(run("ic_gemm_w4a16_ws", *a16, ws=ws), run("ic_gemm_w4a16", *a16, ws=None))
