@@ -152,10 +152,11 @@ struct RqLds {
   // Waves per SIMD that the LDS admits, which the registers then have to (the
   // compiler otherwise took up to 184 and left one workgroup of two or three).
   // At most three (168 registers; four spill), four where two seven-wave
-  // workgroups need them.
+  // workgroups need them, two for the three tiles of unrotated normalised rows.
   static constexpr int kWgs = occ(XROT ? kXbTight : kXbPad, DBR ? 2 : 1);
   static constexpr int kWaves = (kWgs * (TH / 64) + 3) / 4;
-  static constexpr int kMinWaves = kWaves < 3 ? (kWaves < 1 ? 1 : kWaves) : (TH == 448 && NT == 1 && NORM == 0 ? kWaves : 3);
+  static constexpr int kCap = LOG4R == 0 && NORM != 0 && NT == 3 ? 2 : 3;
+  static constexpr int kMinWaves = kWaves < kCap ? (kWaves < 1 ? 1 : kWaves) : (TH == 448 && NT == 1 && NORM == 0 ? kWaves : kCap);
 };
 
 // Three instantiation sets (VAR): kRqPlain (no SmoothRot factors, no perm),
@@ -844,7 +845,12 @@ hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
 // Two tiles of three or four waves instead where one wide tile leaves a single
 // workgroup per CU or too few registers: eight waves (4608 x 8192 48.6 against
 // 52.9), seven and up to six with a norm (LayerNorm, 4608 x 5120: 46.8 against
-// 79 on five waves), and five or six unrotated (no LDS exchange to shorten).
+// 79 on five waves), five or six unrotated (no LDS exchange to shorten), and
+// six where one wide tile leaves a single workgroup per CU: without factors and
+// perm, or at R = 1024 (8192 x 6144, R = 256, f16 without factors 64.1 -> 43.0,
+// bf16 67.8 -> 48.0; R = 1024 with both 87.5 -> 68.5 and 94.0 -> 73.6).  Three
+// tiles of four waves for normalised unrotated rows of nine to twelve thousand
+// values (LayerNorm, 8192 x 10240: 142 -> 123 against twelve waves).
 template <int DT, int LOG4R, int VAR, int NORM = 0, bool QUANT = true>
 hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
 #define IC_RQ(NT, TH) return launch_fast_t<DT, LOG4R, NT, VAR, TH, NORM, QUANT>(a, st)
@@ -858,7 +864,7 @@ hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
         if constexpr (NORM == 0 && LOG4R >= 3) IC_RQ(1, 320);
         IC_RQ(2, 192);
       case 6:
-        if constexpr (NORM == 0 && LOG4R >= 3) IC_RQ(1, 384);
+        if constexpr (NORM == 0 && VAR != kRqPlain && (LOG4R == 3 || LOG4R == 4)) IC_RQ(1, 384);
         IC_RQ(2, 192);
       case 7:
         if constexpr (NORM == 0 && RqLds<DT, LOG4R, 1, VAR, 448, NORM>::kWgs >= 2) IC_RQ(1, 448);
@@ -867,7 +873,9 @@ hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
       case 9:
       case 10:
       case 11:
-      case 12: IC_RQ(1, 768);
+      case 12:
+        if constexpr (LOG4R == 0 && NORM != 0) IC_RQ(3, 256);
+        IC_RQ(1, 768);
       case 13:
       case 14:
         if constexpr (LOG4R == 5) IC_RQ(2, 448);
