@@ -349,6 +349,7 @@ def rotate_quantize(x: torch.Tensor, *, rot_size: int = 0, w_in: int | None = No
 
 def _fused_limit(dt: int) -> int:
     """Widest row the single-pass prep kernels hold."""
+    lib()  # raises where the library is not loaded
     return _max_fused_row // (2 if dt == IC_DTYPE_F32 else 1)
 
 

@@ -100,3 +100,16 @@ def test_dynamic_quantize_cpu_branch_is_reference_semantics(rt):
     ref_s = x.abs().amax(dim=1).clamp(min=1e-8) / 127.0
     assert torch.equal(s, ref_s)
     assert torch.equal(q, (x / ref_s[:, None]).round().clamp(-128, 127).to(torch.int8))
+
+
+@pytest.mark.parametrize("entry", ["rotate_quantize", "prepare_activation", "norm_rotate_quantize"])
+def test_missing_library_is_named(rt, monkeypatch, entry):
+    """Without the kernel library the preparation entry points raise the error
+    that names it (the widest fused row comes from the library too)."""
+    import torch
+
+    monkeypatch.setattr(rt, "_lib", None)
+    monkeypatch.setattr(rt, "_max_fused_row", 0)
+    monkeypatch.setattr(rt, "_need_cuda", lambda *tensors: None)
+    with pytest.raises(RuntimeError, match="not loaded"):
+        getattr(rt, entry)(torch.zeros(2, 64, dtype=torch.float16))
