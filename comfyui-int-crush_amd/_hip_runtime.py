@@ -92,6 +92,7 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "ic_gemm_w4a16_splitk_bytes": ([_L, _L, _L, _L], _L),
     "ic_gemm_w4a16_ws": ([_P, _I, _L, _L, _L, _P, _L, _L, _P, _L, _P, _I, _P, _L, _P, _L, _P], _I),
     "ic_gemm_w4a16_staged_ws": ([_P, _I, _L, _L, _L, _P, _L, _P, _L, _P, _I, _P, _L, _P, _L, _P], _I),
+    "ic_gemm_route": ([_I, _L, _L, _L, _L, _L, _P], _I),
     "ic_unpack_int4_to_int8": ([_P, _L, _L, _L, _P, _L, _P], _I),
     "ic_unpack_int4_to_float": ([_P, _P, _L, _L, _L, _L, _P, _I, _L, _P], _I),
     "ic_f6_activation_bytes": ([_L, _L], _L),
@@ -587,6 +588,25 @@ def _w16_workspace(M: int, N: int, K: int, G: int, device) -> tuple[torch.Tensor
     if nb <= 0:
         return None, 0
     return torch.empty(nb, dtype=torch.uint8, device=device), nb
+
+
+IC_WEIGHTS_I8, IC_WEIGHTS_I4, IC_WEIGHTS_W4A16 = 0, 1, 2
+_ROUTES = ("scalar", "gemv", "tiles", "big", "small")  # IC_ROUTE_*
+
+
+def gemm_route(weights: int, M: int, N: int, K: int, G: int = 1,
+               workspace_bytes: int | None = None) -> tuple[str, int, int, int]:
+    """(kernel, tile rows, tile columns, K slices) of a GEMM on aligned operands
+    with a 16-bit output (ic_gemm_route); workspace_bytes: by default what the
+    callables here allocate for the shape."""
+    if workspace_bytes is None:
+        if weights == IC_WEIGHTS_W4A16:
+            workspace_bytes = lib().ic_gemm_w4a16_splitk_bytes(M, N, K, G)
+        else:
+            workspace_bytes = lib().ic_gemm_splitk_bytes(M, N, K, G, int(weights == IC_WEIGHTS_I4))
+    r = (ctypes.c_int32 * 4)()
+    _call("ic_gemm_route", weights, M, N, K, G, workspace_bytes, r)
+    return _ROUTES[r[0]], r[1], r[2], r[3]
 
 
 # Epilogue activation codes (kernels/triton_int8_gemm.py:24-27 for 0-2).

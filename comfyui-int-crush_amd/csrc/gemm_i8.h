@@ -934,51 +934,74 @@ double tile_us(const GemmArgs& g, bool grouped, const TileShape& t, int S) {
 // launch chosen otherwise, in S0 slices).  Grouped launches keep its slices:
 // a slice boundary moves the order of the fp32 fold, and the outputs of a
 // shape do not depend on the kernel (nor on the output type, whose f32 form
-// only the other tiles write).  Per-row sums are exact in any slices.  The
-// reduction loads 16 bytes of a workspace: one that is not aligned to them
-// leaves a launch unsplit, or on the other tiles.
+// only the other tiles write).  Per-row sums are exact in any slices, up to
+// the number splitk_plan gives the shape, whose workspace ic_gemm_splitk_bytes
+// states.  The reduction loads 16 bytes of a workspace: one that is not
+// aligned to them leaves a launch unsplit, or on the other tiles.
 bool mid_pick(const GemmArgs& g, int mode, bool grouped, int S0, double base, MidPlan& p) {
   const bool ws_ok = g.ws != nullptr && (((uintptr_t)g.ws) & 15) == 0;
   if (!mid_rounds_ok(g.M, g.N) || (grouped && S0 > 1 && !ws_ok)) return false;
-  const int64_t mn4 = (int64_t)g.M * g.N * 4;
-  const int64_t fit = ws_ok ? g.ws_bytes / mn4 : 0;
-  const int most = fit > 16 ? 16 : (fit < 1 ? 1 : (int)fit);
-  p = grouped ? mid_plan(mode, g.M, g.N, g.K / kBK, S0, S0) : mid_plan(mode, g.M, g.N, g.K / kBK, 1, most);
+  if (grouped) {
+    p = mid_plan(mode, g.M, g.N, g.K / kBK, S0, S0);
+  } else {
+    const int64_t fit = ws_ok ? g.ws_bytes / ((int64_t)g.M * g.N * 4) : 0;
+    const int planned = fit > 1 ? splitk_plan(g, false) : 1;
+    p = mid_plan(mode, g.M, g.N, g.K / kBK, 1, fit < planned ? (int)fit : planned);
+  }
   return p.us < base;
 }
-// Groups of 64 or 32 columns, against the big tile; never split.
-bool mid_pick_unsplit(const GemmArgs& g, int mode, MidPlan& p) {
-  if (!mid_rounds_ok(g.M, g.N)) return false;
-  p = mid_plan(mode, g.M, g.N, g.K / kBK, 1, 1);
-  return p.us < big_us(mode, big_rows(g), g.M, g.N, g.K / kBK);
+
+// The kernel of a launch with a 16-bit output: small tiles, big tiles or, where
+// neither leads or the output is not aligned for them, the tile kernel.
+enum RouteKind { kTiles, kBig, kMid };
+struct Route { RouteKind kind; int mode; TileShape tile; int S; MidPlan mid; };
+
+// whole 128-column blocks per group, or per-row scales
+Route route_of(const GemmArgs& g, bool grouped) {
+  const int mode = grouped ? (g.int4 ? big::G128 : big::G128I8) : (g.int4 ? big::ROW4 : big::ROW8);
+  Route r{kTiles, mode, tile_choice(g, grouped), 1, {}};
+  const bool use_big = grouped ? big_tile_ok(g) : big_row_ok(g);
+  // as launch_mfma splits it
+  if (g.ws != nullptr && !use_big) r.S = splitk_plan(g, grouped);
+  if (g.ws_bytes < (int64_t)r.S * g.M * g.N * 4) r.S = 1;
+  if (big_out_ok(g)) {
+    const double base = use_big ? big_us(mode, big_rows(g), g.M, g.N, g.K / kBK) : tile_us(g, grouped, r.tile, r.S);
+    if (mid_pick(g, mode, grouped, r.S, base, r.mid)) r.kind = kMid;
+  }
+  if (r.kind == kTiles && use_big) r.kind = kBig;
+  return r;
 }
-hipError_t launch_mid_any(const GemmArgs& g, int mode, const MidPlan& p, hipStream_t st) {
-  if (!g.int4) return ic_launch_mid_i8(g, mode, p.tile, p.S, st);
-  return g.kil ? ic_launch_mid_kil(g, mode, p.tile, p.S, st) : ic_launch_mid_i4(g, mode, p.tile, p.S, st);
+// Groups of 64 or 32 columns: small or big tiles, never split.
+Route route_of_small_groups(const GemmArgs& g, int mode) {
+  Route r{kBig, mode, {}, 1, {}};
+  if (mid_rounds_ok(g.M, g.N)) {
+    r.mid = mid_plan(mode, g.M, g.N, g.K / kBK, 1, 1);
+    if (r.mid.us < big_us(mode, big_rows(g), g.M, g.N, g.K / kBK)) r.kind = kMid;
+  }
+  return r;
+}
+hipError_t launch_mid_any(const GemmArgs& g, const Route& r, hipStream_t st) {
+  if (!g.int4) return ic_launch_mid_i8(g, r.mode, r.mid.tile, r.mid.S, st);
+  return g.kil ? ic_launch_mid_kil(g, r.mode, r.mid.tile, r.mid.S, st)
+               : ic_launch_mid_i4(g, r.mode, r.mid.tile, r.mid.S, st);
+}
+template <int MODE, bool EPI>
+hipError_t launch_small_groups(const GemmArgs& g, hipStream_t st) {
+  const Route r = route_of_small_groups(g, MODE);
+  if (r.kind == kMid) return launch_mid_any(g, r, st);
+  if (g.out_dt == IC_DTYPE_F16) return launch_big<IC_DTYPE_F16, EPI, MODE>(g, st);
+  return launch_big<IC_DTYPE_BF16, EPI, MODE>(g, st);
 }
 
 template <bool INT4, int GS, int OUT_DT, bool ACC, bool EPI>
 hipError_t pick_tile(const GemmArgs& g, hipStream_t st) {
-  const TileShape t = tile_choice(g, GS != 0);
   if constexpr (!ACC && OUT_DT != IC_DTYPE_F32) {
-    if (g.C != nullptr && big_out_ok(g)) {
-      constexpr int mode = GS != 0 ? (INT4 ? big::G128 : big::G128I8) : (INT4 ? big::ROW4 : big::ROW8);
-      const bool use_big = GS != 0 ? big_tile_ok(g) : big_row_ok(g);
-      // as launch_mfma splits it
-      int S = g.ws != nullptr && !use_big ? splitk_plan(g, GS != 0) : 1;
-      if (g.ws_bytes < (int64_t)S * g.M * g.N * 4) S = 1;
-      MidPlan p;
-      if (mid_pick(g, mode, GS != 0, S, use_big ? big_us(mode, big_rows(g), g.M, g.N, g.K / kBK) : tile_us(g, GS != 0, t, S), p))
-        return launch_mid_any(g, mode, p, st);
-    }
+    constexpr int mode = GS != 0 ? (INT4 ? big::G128 : big::G128I8) : (INT4 ? big::ROW4 : big::ROW8);
+    const Route r = route_of(g, GS != 0);
+    if (r.kind == kMid) return launch_mid_any(g, r, st);
+    if (r.kind == kBig) return launch_big<OUT_DT, EPI, mode>(g, st);
   }
-  if constexpr (GS != 0 && !ACC && OUT_DT != IC_DTYPE_F32) {
-    // grouped packed INT4, or grouped int8 weights (INT4 unpacked to bytes)
-    if (big_tile_ok(g)) return launch_big<OUT_DT, EPI, INT4 ? big::G128 : big::G128I8>(g, st);
-  }
-  if constexpr (GS == 0 && !ACC && OUT_DT != IC_DTYPE_F32) {
-    if (big_row_ok(g)) return launch_big<OUT_DT, EPI, INT4 ? big::ROW4 : big::ROW8>(g, st);
-  }
+  const TileShape t = tile_choice(g, GS != 0);
   if constexpr (!INT4 && GS == 0) {
     if (t.bm == 256 && t.bn == 192) return launch_mfma<Tile<256, 192, 4, 2, false, 0>, OUT_DT, ACC, EPI>(g, st);
     if (t.bm == 256) return launch_mfma<Tile<256, 256, 2, 2, false, 0>, OUT_DT, ACC, EPI>(g, st);
@@ -1112,17 +1135,11 @@ int run_gemm_t(GemmArgs g, hipStream_t st, const char* who, bool force_generic) 
   if (!force_generic && big64_ok(g, gsize)) {
     // groups of 64 (or an odd multiple of 64) columns: the 288 x 192 kernel
     // folding each 64-K step, or the small tiles, at any M
-    MidPlan p;
-    if (mid_pick_unsplit(g, big::G64, p)) e = launch_mid_any(g, big::G64, p, st);
-    else if (g.out_dt == IC_DTYPE_F16) e = launch_big<IC_DTYPE_F16, EPI, big::G64>(g, st);
-    else e = launch_big<IC_DTYPE_BF16, EPI, big::G64>(g, st);
+    e = launch_small_groups<big::G64, EPI>(g, st);
   } else if (!force_generic && big32_ok(g, gsize)) {
-    // groups of 32 (or an odd multiple of 32) columns: the same kernel folding
+    // groups of 32 (or an odd multiple of 32) columns: the same kernels folding
     // each 32-column half step
-    MidPlan p;
-    if (mid_pick_unsplit(g, big::G32, p)) e = launch_mid_any(g, big::G32, p, st);
-    else if (g.out_dt == IC_DTYPE_F16) e = launch_big<IC_DTYPE_F16, EPI, big::G32>(g, st);
-    else e = launch_big<IC_DTYPE_BF16, EPI, big::G32>(g, st);
+    e = launch_small_groups<big::G32, EPI>(g, st);
   } else if (!force_generic && mfma_shape_ok(g, gsize)) {
     if constexpr (EPI) {
       // the epilogue options never come with the debug accumulator output

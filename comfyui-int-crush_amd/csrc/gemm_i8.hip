@@ -93,6 +93,47 @@ int64_t ic_gemm_splitk_bytes(int64_t M, int64_t N, int64_t K, int64_t num_groups
   return S > 1 ? (int64_t)S * M * N * 4 : 0;
 }
 
+int ic_gemm_route(int weights, int64_t M, int64_t N, int64_t K, int64_t num_groups, int64_t workspace_bytes,
+                  int32_t* route) {
+  const char* who = "ic_gemm_route";
+  if (route == nullptr || weights < IC_WEIGHTS_I8 || weights > IC_WEIGHTS_W4A16 || M < 1 || N < 1 || K < 1 ||
+      num_groups < 1 || K % num_groups != 0 || workspace_bytes < 0 || M * N > (1LL << 31))
+    return ic_set_error(IC_ERR_INVALID_ARG, "%s: bad shape M=%lld N=%lld K=%lld groups=%lld weights=%d", who,
+                        (long long)M, (long long)N, (long long)K, (long long)num_groups, weights);
+  if (weights == IC_WEIGHTS_W4A16) {
+    ic_w4a16_route(M, N, K, num_groups, workspace_bytes, route);
+    return IC_OK;
+  }
+  // stands for aligned operands, outputs and workspace; nothing reads it
+  char* const aligned = (char*)256;
+  const bool int4 = weights == IC_WEIGHTS_I4;
+  const int64_t ldo = (N + 7) / 8 * 8;
+  GemmArgs g{(const int8_t*)aligned, (K + 15) / 16 * 16, (const uint8_t*)aligned, (K + 31) / 32 * (int4 ? 16 : 32),
+             nullptr, nullptr, (int)num_groups, nullptr, 0, aligned, IC_DTYPE_BF16, ldo, (int)M, (int)N, (int)K,
+             nullptr, int4, workspace_bytes > 0 ? aligned : nullptr, workspace_bytes};
+  const auto put = [route](int kind, int bm, int bn, int S) {
+    route[0] = kind; route[1] = bm; route[2] = bn; route[3] = S;
+  };
+  const int gsize = (int)(K / num_groups);
+  if (ic_gemv_applicable(M, K, g.A, g.lda, g.B, g.ldb) &&
+      (int4 ? ic_gemv_w4a8_groups_ok(M, K, num_groups) : num_groups == 1)) {
+    put(IC_ROUTE_GEMV, 0, 0, 1);
+    return IC_OK;
+  }
+  Route r;
+  if (big64_ok(g, gsize)) r = route_of_small_groups(g, big::G64);
+  else if (big32_ok(g, gsize)) r = route_of_small_groups(g, big::G32);
+  else if (mfma_shape_ok(g, gsize)) r = route_of(g, num_groups > 1);
+  else {
+    put(IC_ROUTE_SCALAR, 0, 0, 1);
+    return IC_OK;
+  }
+  if (r.kind == kMid) put(IC_ROUTE_SMALL_TILES, kMidTile[r.mid.tile].bm, kMidTile[r.mid.tile].bn, r.mid.S);
+  else if (r.kind == kBig) put(IC_ROUTE_BIG_TILES, 32 * big_rows(g), big::BN, 1);
+  else put(IC_ROUTE_TILES, r.tile.bm, r.tile.bn, r.S);
+  return IC_OK;
+}
+
 int ic_gemm_w8a8_ex(const int8_t* xq, int64_t M, int64_t K, int64_t ldx, const int8_t* w, int64_t N, int64_t ldw,
                     const float* s_a, const float* s_w, const void* bias, int bias_dtype, int activation,
                     const void* residual, int residual_dtype, int64_t ldr, void* out, int out_dtype, int64_t ldo,

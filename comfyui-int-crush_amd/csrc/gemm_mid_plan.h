@@ -76,3 +76,5 @@ hipError_t ic_launch_mid_i4(const ic_gemm::GemmArgs& g, int mode, int tile, int 
 hipError_t ic_launch_mid_kil(const ic_gemm::GemmArgs& g, int mode, int tile, int S, hipStream_t st);
 hipError_t ic_launch_mid_i8(const ic_gemm::GemmArgs& g, int mode, int tile, int S, hipStream_t st);
 hipError_t ic_launch_mid_w16(const ic_gemm::GemmArgs& g, int tile, int S, hipStream_t st);
+// ic_gemm_route for W4A16 (gemm_w4a16.hip)
+void ic_w4a16_route(int64_t M, int64_t N, int64_t K, int64_t num_groups, int64_t ws_bytes, int32_t* route);

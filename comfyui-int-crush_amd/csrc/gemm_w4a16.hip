@@ -341,9 +341,8 @@ hipError_t launch_w4a16_big_t(const u16* A, int64_t lda, const uint8_t* B, int64
 // us, bit-identical; forced onto shapes where they take more rounds x area,
 // 4608 x 3072 x 3072 75 -> 79 us, 4096 x 5120 x 5120 216 -> 258 us).
 constexpr int kW16WidePct = 95;
-template <int DT, int NARROW, int WIDE, bool STG>
-hipError_t launch_w4a16_big_m(const u16* A, int64_t lda, const uint8_t* B, int64_t ldb, const float* s_w, int G,
-                              const void* bias, int bias_dt, u16* C, int64_t ldc, int M, int N, int K, hipStream_t st) {
+struct W16Big { int tmb; bool wide; };  // 32 tmb rows on 192 or 256 columns
+W16Big w16_big_pick(int64_t M, int64_t N) {
   const int64_t cus = ic_num_cus();
   auto cost = [&](int bm, int bn, int pct) {
     const int64_t t = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
@@ -351,15 +350,22 @@ hipError_t launch_w4a16_big_m(const u16* A, int64_t lda, const uint8_t* B, int64
   };
   const int64_t c9 = cost(288, 192, 100), c8 = cost(256, 192, 105), c10 = cost(320, 192, 99);
   const int64_t w9 = cost(288, 256, kW16WidePct), w8 = cost(256, 256, kW16WidePct * 105 / 100);
-  const int64_t cn = std::min(c9, std::min(c8, c10)), cw = std::min(w9, w8);
-  if (cw < cn) {
-    if (w8 < w9)
+  if (std::min(w9, w8) < std::min(c9, std::min(c8, c10))) return {w8 < w9 ? 8 : 9, true};
+  if (c8 < c9 && c8 <= c10) return {8, false};
+  return {c10 < c9 ? 10 : 9, false};
+}
+template <int DT, int NARROW, int WIDE, bool STG>
+hipError_t launch_w4a16_big_m(const u16* A, int64_t lda, const uint8_t* B, int64_t ldb, const float* s_w, int G,
+                              const void* bias, int bias_dt, u16* C, int64_t ldc, int M, int N, int K, hipStream_t st) {
+  const W16Big p = w16_big_pick(M, N);
+  if (p.wide) {
+    if (p.tmb == 8)
       return launch_w4a16_big_t<DT, 8, WIDE, STG>(A, lda, B, ldb, s_w, G, bias, bias_dt, C, ldc, M, N, K, st);
     return launch_w4a16_big_t<DT, 9, WIDE, STG>(A, lda, B, ldb, s_w, G, bias, bias_dt, C, ldc, M, N, K, st);
   }
-  if (c8 < c9 && c8 <= c10)
+  if (p.tmb == 8)
     return launch_w4a16_big_t<DT, 8, NARROW, STG>(A, lda, B, ldb, s_w, G, bias, bias_dt, C, ldc, M, N, K, st);
-  if (c10 < c9)
+  if (p.tmb == 10)
     return launch_w4a16_big_t<DT, 10, NARROW, STG>(A, lda, B, ldb, s_w, G, bias, bias_dt, C, ldc, M, N, K, st);
   return launch_w4a16_big_t<DT, 9, NARROW, STG>(A, lda, B, ldb, s_w, G, bias, bias_dt, C, ldc, M, N, K, st);
 }
@@ -410,6 +416,22 @@ int w16_max_splits(int64_t M, int64_t N, const void* ws, int64_t ws_bytes) {
   return fit > kW16MaxSplits ? kW16MaxSplits : (fit < 1 ? 1 : (int)fit);
 }
 
+// By rounds of workgroups x tile area x relative cost per output: 384 x 192
+// tiles (wave tiles of 96 x 96, a two-slot ring) where they fill the CUs in
+// fewer rounds than 256 x 256, e.g. 4608 x 12288: 768 tiles, three rounds,
+// against 864 of 256 x 256 (four).  Per output they cost ~5 % more than
+// 256 x 256 (more activation bytes per stage), but dequantize fewer weights
+// per output than the 192 x 384 tile of the same area, which measured 11 %
+// slower at that shape.
+bool w4a16_tall(int64_t M, int64_t N) {
+  const int64_t cus = ic_num_cus();
+  auto cost = [&](int bm, int bn, int pct) {
+    const int64_t t = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    return (t + cus - 1) / cus * bm * bn * pct;
+  };
+  return cost(384, 192, 105) < cost(256, 256, 100);
+}
+
 template <int DT>
 hipError_t run_w4a16(const u16* A, int64_t lda, const uint8_t* B, int64_t ldb, const float* s_w, int G,
                      int gsize, const void* bias, int bias_dt, u16* C, int64_t ldc, int M, int N, int K,
@@ -421,17 +443,7 @@ hipError_t run_w4a16(const u16* A, int64_t lda, const uint8_t* B, int64_t ldb, c
   if (mfma_ok) {
     if (M > 128 && big_ok) return launch_w4a16_big<DT>(A, lda, B, ldb, s_w, G, bias, bias_dt, C, ldc, M, N, K, st);
     if (M > 128) {
-      // rounds of workgroups x tile area x relative cost per output: 384 x 192 tiles (wave tiles of
-      // 96 x 96, a two-slot ring) where they fill the CUs in fewer rounds, e.g. 4608 x 12288: 768
-      // tiles, three rounds, against 864 of 256 x 256 (four).  Per output they cost ~5 % more than
-      // 256 x 256 (more activation bytes per stage), but dequantize fewer weights per output than
-      // the 192 x 384 tile of the same area, which measured 11 % slower at that shape.
-      const int64_t cus = ic_num_cus();
-      auto cost = [&](int bm, int bn, int pct) {
-        const int64_t t = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        return (t + cus - 1) / cus * bm * bn * pct;
-      };
-      if (cost(384, 192, 105) < cost(256, 256, 100))
+      if (w4a16_tall(M, N))
         return launch_w4a16<WTile<384, 192, 4, 2>, DT>(A, lda, B, ldb, s_w, G, gsize, bias, bias_dt, C, ldc, M, N, K, st);
       return launch_w4a16<WTile<256, 256, 2, 3>, DT>(A, lda, B, ldb, s_w, G, gsize, bias, bias_dt, C, ldc, M, N, K, st);
     }
@@ -485,6 +497,32 @@ __global__ void w4a16_stage_s_kernel(const float* __restrict__ S, float* __restr
 }
 
 }  // namespace
+
+// The routes of run_w4a16 (and, above 128 rows, of the staged layout) for
+// 16-byte aligned operands and workspace.
+void ic_w4a16_route(int64_t M, int64_t N, int64_t K, int64_t num_groups, int64_t ws_bytes, int32_t* route) {
+  const auto put = [route](int kind, int bm, int bn, int S) {
+    route[0] = kind; route[1] = bm; route[2] = bn; route[3] = S;
+  };
+  const int64_t gsize = K / num_groups;
+  const void* const aligned = (const void*)256;
+  if (ic_gemv_applicable(M, K, aligned, 0, aligned, 0) && (num_groups == 1 || gsize % 32 == 0))
+    return put(IC_ROUTE_GEMV, 0, 0, 1);
+  const bool mfma_ok = K % 64 == 0 && (num_groups == 1 || gsize % 32 == 0) && 384 * K * 2 < (1LL << 31) &&
+                       N * num_groups * 4 < (1LL << 31);
+  if (!mfma_ok) return put(IC_ROUTE_SCALAR, 0, 0, 1);
+  if ((num_groups == 1 || gsize % 64 == 0) && N % 8 == 0) {
+    const MidPlan p = w16_plan(M, N, K, w16_max_splits(M, N, ws_bytes > 0 ? aligned : nullptr, ws_bytes));
+    if (p.S > 0) return put(IC_ROUTE_SMALL_TILES, kMidTile[p.tile].bm, kMidTile[p.tile].bn, p.S);
+    if (M > 128) {
+      const W16Big b = w16_big_pick(M, N);
+      return put(IC_ROUTE_BIG_TILES, 32 * b.tmb, b.wide ? 256 : big::BN, 1);
+    }
+  }
+  if (M <= 128) return put(IC_ROUTE_TILES, 128, 256, 1);
+  if (w4a16_tall(M, N)) return put(IC_ROUTE_TILES, 384, 192, 1);
+  put(IC_ROUTE_TILES, 256, 256, 1);
+}
 
 extern "C" {
 

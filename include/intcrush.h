@@ -177,10 +177,9 @@ int ic_gemm_w4a8(const int8_t* xq, int64_t M, int64_t K, int64_t ldx, const uint
  * only in the order of the fp32 additions.  ic_gemm_splitk_bytes returns the
  * most workspace a launch of that shape uses (0: no split; then workspace may
  * be null); a smaller workspace than that runs on fewer slices or unsplit, as
- * one not aligned to 16 bytes may.
- * Launches with 16-bit, 16-byte aligned outputs may take small tiles instead,
- * in fewer slices or none.  The library itself
- * never allocates.
+ * one not aligned to 16 bytes may.  Launches with 16-bit, 16-byte aligned
+ * outputs may take small tiles instead, in as many slices, fewer or none.  The
+ * library itself never allocates.
  */
 int64_t ic_gemm_splitk_bytes(int64_t M, int64_t N, int64_t K, int64_t num_groups, int int4);
 int ic_gemm_w8a8_ws(const int8_t* xq, int64_t M, int64_t K, int64_t ldx, const int8_t* w, int64_t N,
@@ -355,6 +354,26 @@ int ic_gemm_w4a16_ws(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx
 int ic_gemm_w4a16_staged_ws(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w_staged,
                             int64_t N, const float* s_staged, int64_t num_groups, const void* bias, int bias_dtype,
                             void* out, int64_t ldo, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
+ * The kernel that the GEMM entry points above take for a shape, on the current
+ * device: for 16-byte aligned operands and output rows, a 16-bit output and a
+ * workspace of workspace_bytes (0: none).  weights: IC_WEIGHTS_*, int8 with
+ * num_groups > 1 being the unpacked INT4 form; W4A16 the packed and, above 128
+ * rows, the staged layout.  route receives the kind (IC_ROUTE_*), the rows and
+ * columns of an output tile (0 without tiles) and the K slices.  Host
+ * arithmetic only; no reference counterpart.
+ */
+#define IC_WEIGHTS_I8 0
+#define IC_WEIGHTS_I4 1
+#define IC_WEIGHTS_W4A16 2
+#define IC_ROUTE_SCALAR 0
+#define IC_ROUTE_GEMV 1
+#define IC_ROUTE_TILES 2
+#define IC_ROUTE_BIG_TILES 3
+#define IC_ROUTE_SMALL_TILES 4
+int ic_gemm_route(int weights, int64_t M, int64_t N, int64_t K, int64_t num_groups, int64_t workspace_bytes,
+                  int32_t* route);
 
 /*
  * Small-batch GEMV forms (1 <= M <= IC_GEMV_MAX_M tokens, K a multiple of 128

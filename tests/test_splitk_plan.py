@@ -26,3 +26,25 @@ def test_splitk_plan(rt, M, N, K, G, int4, split):
     assert (nb > 0) == split, nb
     if split:
         assert nb % (4 * M * N) == 0 and 2 <= nb // (4 * M * N) <= 16
+
+
+def _shapes():
+    return [(M, N, K) for M in (17, 64, 77, 128, 200, 232, 300, 366, 512, 1024)
+            for N, K in ((3072, 3072), (5920, 7424), (3856, 7040), (3072, 12288), (1024, 1024))]
+
+
+def test_no_launch_uses_more_than_the_stated_workspace(rt):
+    """ic_gemm_splitk_bytes (ic_gemm_w4a16_splitk_bytes) is the most workspace
+    a launch uses: a larger one does not raise the number of slices."""
+    for M, N, K in _shapes():
+        for weights, G in ((0, 1), (1, 1), (1, K // 128), (0, K // 128), (2, K // 128)):
+            stated = (rt.lib().ic_gemm_w4a16_splitk_bytes(M, N, K, G) if weights == 2 else
+                      rt.lib().ic_gemm_splitk_bytes(M, N, K, G, weights))
+            route = rt.gemm_route(weights, M, N, K, G, workspace_bytes=64 * M * N * 4)
+            assert route[3] <= max(1, stated // (4 * M * N)), (weights, M, N, K, G, route)
+
+
+def test_route_argument_validation(rt):
+    for bad in ((3, 1, 1, 1, 1), (0, 0, 8, 128, 1), (0, 8, 8, 128, 3), (1, 1 << 20, 1 << 20, 128, 1)):
+        with pytest.raises(RuntimeError):
+            rt.gemm_route(*bad, workspace_bytes=0)
