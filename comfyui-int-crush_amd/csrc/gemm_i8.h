@@ -945,8 +945,8 @@ bool mid_pick(const GemmArgs& g, int mode, bool grouped, int S0, double base, Mi
     p = mid_plan(mode, g.M, g.N, g.K / kBK, S0, S0);
   } else {
     const int64_t fit = ws_ok ? g.ws_bytes / ((int64_t)g.M * g.N * 4) : 0;
-    const int planned = fit > 1 ? splitk_plan(g, false) : 1;
-    p = mid_plan(mode, g.M, g.N, g.K / kBK, 1, fit < planned ? (int)fit : planned);
+    const int most = fit > 1 ? splitk_plan(g, false) : 1;
+    p = mid_plan(mode, g.M, g.N, g.K / kBK, 1, fit > 1 && fit < most ? (int)fit : most);
   }
   return p.us < base;
 }

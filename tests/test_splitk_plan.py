@@ -48,3 +48,12 @@ def test_route_argument_validation(rt):
     for bad in ((3, 1, 1, 1, 1), (0, 0, 8, 128, 1), (0, 8, 8, 128, 3), (1, 1 << 20, 1 << 20, 128, 1)):
         with pytest.raises(RuntimeError):
             rt.gemm_route(*bad, workspace_bytes=0)
+
+
+@pytest.mark.parametrize("weights", [0, 1, 2])
+def test_small_tiles_without_a_workspace(rt, weights):
+    """Launches of few tiles take the small ones, unsplit, also where there is no
+    workspace (or the shape's plan asks for none)."""
+    for M, N, K in ((64, 1024, 1024), (200, 1024, 1024), (256, 4096, 1152)):
+        kind, _, _, S = rt.gemm_route(weights, M, N, K, 1, workspace_bytes=0)
+        assert (kind, S) == ("small", 1), (M, N, K)
