@@ -910,24 +910,21 @@ hipError_t launch_big(const GemmArgs& g, hipStream_t st) {
   }
 }
 
-// Estimated microseconds of the launch the rules above choose (model and
-// constants as in gemm_mid_plan.h): rounds of workgroups x stages x the
-// stage time of a tile, 256 x 192 for the big kernel and scaled with its area.
+// Estimated microseconds of the launch the rules above choose (gemm_mid_plan.h
+// has the model and its constants).
 double big_us(int mode, int tmb, int64_t M, int64_t N, int KT) {
-  constexpr double stage[6] = {1.5, 1.8, 1.1, 1.1, 3.5, 1.6};  // by weight mode G128 ... G128I8
+  const LargeCost& c = kLargeCost[mode];
   const int64_t cus = ic_num_cus();
   const int64_t tiles = ((M + 32 * tmb - 1) / (32 * tmb)) * ((N + big::BN - 1) / big::BN);
-  return (double)((tiles + cus - 1) / cus) * (KT * stage[mode] * tmb / 8.0 + 4.0) + 5.0;
+  return c.fixed + (double)((tiles + cus - 1) / cus) * (KT * c.stage * tmb / 8.0 + c.end);
 }
-double tile_us(const GemmArgs& g, bool grouped, const TileShape& t, int S) {
+double tile_us(const GemmArgs& g, int mode, const TileShape& t, int S) {
+  const LargeCost& c = kLargeCost[mode];
   const int64_t cus = ic_num_cus(), area = (int64_t)t.bm * t.bn / 16384;  // of 128 x 128
   const int64_t n = (int64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn) * S;
-  // one 128 x 128 stage, and each further 128 x 128 of a larger tile
-  const double one = g.int4 ? (grouped ? 0.85 : 0.70) : (grouped ? 0.60 : 0.55);
-  const double more = g.int4 ? (grouped ? 0.30 : 0.25) : (grouped ? 0.45 : 0.35);
   const int KT = g.K / kBK;
-  return kMidFixed + 1.0 + (double)((n + cus - 1) / cus) * ((KT + S - 1) / S) * (one + more * (area - 1)) +
-         (S > 1 ? kMidReduce + (double)S * g.M * g.N * 8.0 / kMidBytesPerUs : 0.0);
+  return c.t_fixed + (double)((n + cus - 1) / cus) * ((KT + S - 1) / S * (c.one + c.more * (area - 1)) + c.t_end) +
+         (S > 1 ? c.reduce + (double)S * g.M * g.N * 8.0 / c.bytes : 0.0);
 }
 
 // The small tiles instead, where their estimate is below `base` (that of the
@@ -965,7 +962,7 @@ Route route_of(const GemmArgs& g, bool grouped) {
   if (g.ws != nullptr && !use_big) r.S = splitk_plan(g, grouped);
   if (g.ws_bytes < (int64_t)r.S * g.M * g.N * 4) r.S = 1;
   if (big_out_ok(g)) {
-    const double base = use_big ? big_us(mode, big_rows(g), g.M, g.N, g.K / kBK) : tile_us(g, grouped, r.tile, r.S);
+    const double base = use_big ? big_us(mode, big_rows(g), g.M, g.N, g.K / kBK) : tile_us(g, mode, r.tile, r.S);
     if (mid_pick(g, mode, grouped, r.S, base, r.mid)) r.kind = kMid;
   }
   if (r.kind == kTiles && use_big) r.kind = kBig;

@@ -372,11 +372,14 @@ __global__ __launch_bounds__(mid::kMT, 2) void gemm_mid_kernel(
 // workgroups share a CU's 160 KB of LDS.
 template <int T, int MODE>
 using MidCfg = mid::Cfg<kMidTile[T].bm / 32, kMidTile[T].bn / 32,
-                        T < 2 ? 4 : (T == 3 && (MODE == big::ROW8 || MODE == big::G128I8) ? 2 : 3), MODE>;
+                        T < 2 ? 4 : (T == 3 && MODE == big::ROW8 ? 2 : 3), MODE>;
 
 template <int T, int MODE, int OUT_DT, bool EPI, bool KIL, bool PART>
 hipError_t launch_mid_k(const ic_gemm::GemmArgs& g, int S, hipStream_t st) {
   using CF = MidCfg<T, MODE>;
+  // LDS goes in 512-byte granules; the registers (at most 116) hold as many workgroups
+  static_assert(kMidCost[MODE].wgs[T] == 0 || kMidCost[MODE].wgs[T] == 163840 / ((CF::lds_bytes + 511) / 512 * 512),
+                "the plan's workgroups per CU");
   const int tiles = ((g.M + CF::BM - 1) / CF::BM) * ((g.N + CF::BN - 1) / CF::BN);
   auto kern = gemm_mid_kernel<CF, OUT_DT, EPI, KIL, PART>;
   static unsigned char lds_set[64];  // per device

@@ -1,22 +1,24 @@
 // Choice of the small-tile kernel (gemm_mid.h) and its K split: host logic
 // shared by the INT8 and W4A16 entry points.
 //
-// Times in microseconds, from launches measured on MI355X (bf16 outputs,
-// weights cycling through three copies).  A tile's stage takes `lat` alone on
-// its CU and `thr` for each workgroup that shares it:
-//   W8A8   512 x 3072 x 3072 (24 stages): 64 x 64 tiles, 384 of them, 12.8 us;
-//          32 x 64 14.4, 128 x 64 15.5, 128 x 128 19.5; 256 x 192 in two
-//          slices 25.4
-//   W8A8   77 x 4096 x 4096: 32 x 64 9.2, 64 x 64 11.4; 128 x 128 in eight
-//          slices 16.5
+// Estimated microseconds, fitted to launches timed on MI355X (bf16 outputs, back
+// to back in a graph, weights cycling through three copies; 566 shapes of 17 to
+// 3072 rows, 1024 to 18432 columns and K 1024 to 14336 per mode, each tile and
+// slice count by itself: 5 to 8 % rms).  A CU takes its workgroups in turns of
+// as many as its LDS holds (`wgs`); in a turn of n a stage takes max(lat, n *
+// thr), and a turn ends with `end` (its epilogue).  Where a tile's stage is
+// bound by the VALU's folds (groups of 64 and 32 columns) the turns do not show
+// and wgs is 0, any number at once.
+//   W4A16  512 x 9216 x 3072: 128 x 64 tiles, three per CU in two turns, 81 us;
+//          256 x 192 tiles 65 (128 x 128: 71)
+//   W4A16  768 x 18432 x 3072: 128 x 128 139; 256 x 256 tiles in one turn 90
+//   W8A8   2048 x 12288 x 3072: 128 x 128 82; 256 x 192 72.6; 512 x 3072 x 3072:
+//          64 x 64 tiles 12.8, 256 x 192 in two slices 25.4
+//   g128   640 x 12288 x 3072: 128 x 64 48; 256 x 192 43
+//   int8 weights in groups, 384 x 18432 x 3072: 64 x 64 54; 256 x 192 43.4
 //   g64    146 x 1312 x 8448: 32 x 64 29.7, 64 x 64 43.1; 256 x 192 125.5
-//   W4A16  63 x 3256 x 3712: 64 x 64 33.8, in four slices 16.5; 128 x 256 68.9
-// The large tiles stay ahead once they fill the CUs (W8A8 1111 x 9216 x 3072:
-// 35.6 against 43.8 us; g128 1357 x 7688 x 2560: 40.7 against 49.4), and past
-// two rounds of them the small ones are not looked at (mid_rounds_ok): the
-// estimates leave out the epilogues' memory time, which weighs on short K
-// (W8A8 19053 x 10992 x 1152 with GELU and a residual: 608 us on 320 x 192
-// tiles, 624 us on 128 x 128).
+// Past two rounds of the large tiles the small ones are not looked at
+// (mid_rounds_ok).
 #pragma once
 #include "gemm_common.h"
 
@@ -26,19 +28,39 @@ struct MidTile { int bm, bn; };
 constexpr int kMidTiles = 4;
 constexpr MidTile kMidTile[kMidTiles] = {{32, 64}, {64, 64}, {128, 64}, {128, 128}};
 
-struct MidCost { double lat[kMidTiles], thr[kMidTiles]; };  // 0: the mode has no such tile
+struct MidCost {
+  double fixed, reduce, bytes;  // of a launch; a split's second kernel, and its partials (8 bytes each) per us
+  int wgs[kMidTiles];
+  double lat[kMidTiles], thr[kMidTiles], end[kMidTiles];  // lat 0: the mode has no such tile
+};
 // by weight mode (big::G128 ... big::W16): 128-K stages, 64-K for W16
 constexpr MidCost kMidCost[7] = {
-    {{0.27, 0.36, 0.55, 0}, {0.175, 0.28, 0.42, 0}},        // G128
-    {{0.39, 0.60, 0.80, 0}, {0.22, 0.33, 0.55, 0}},         // G64
-    {{0.25, 0.32, 0.52, 0}, {0.17, 0.25, 0.38, 0}},         // ROW4
-    {{0.21, 0.265, 0.48, 0.61}, {0.16, 0.21, 0.36, 0.42}},  // ROW8
-    {{0.62, 0.95, 1.40, 0}, {0.40, 0.60, 1.05, 0}},         // G32
-    {{0.30, 0.42, 0.57, 0}, {0.21, 0.26, 0.46, 0}},         // G128I8
-    {{0.48, 0.54, 0.75, 0.98}, {0.27, 0.32, 0.43, 0.65}},   // W16
+    {5.66, 2.35, 3.47e6, {4, 3, 2, 0},
+     {0.22, 0.42, 0.64, 0}, {0.195, 0.243, 0.405, 0}, {0.27, 0.56, 0.98, 0}},  // G128
+    {3.0, 2.5, 5.0e6, {0, 0, 0, 0}, {0.39, 0.60, 0.80, 0}, {0.22, 0.33, 0.55, 0}, {0, 0, 0, 0}},  // G64
+    {4.50, 2.26, 3.26e6, {5, 3, 2, 0},
+     {0.22, 0.28, 0.50, 0}, {0.140, 0.174, 0.358, 0}, {0.36, 0.71, 0.67, 0}},  // ROW4
+    {4.70, 2.94, 4.63e6, {3, 2, 2, 2},
+     {0.19, 0.24, 0.48, 0.77}, {0.167, 0.197, 0.293, 0.423}, {0.10, 0.89, 0.98, 1.51}},  // ROW8
+    {3.0, 2.5, 5.0e6, {0, 0, 0, 0}, {0.62, 0.95, 1.40, 0}, {0.40, 0.60, 1.05, 0}, {0, 0, 0, 0}},  // G32
+    {5.39, 3.41, 5.12e6, {3, 2, 2, 0},
+     {0.23, 0.35, 0.54, 0}, {0.193, 0.258, 0.407, 0}, {0.38, 1.36, 1.33, 0}},  // G128I8
+    {6.06, 3.77, 6.49e6, {6, 3, 2, 2},
+     {0.43, 0.44, 0.72, 0.90}, {0.293, 0.300, 0.409, 0.711}, {0, 0, 0.60, 0.13}},  // W16
 };
-// fixed part of a launch; the second kernel of a split and its partials' round trip
-constexpr double kMidFixed = 3.0, kMidReduce = 2.5, kMidBytesPerUs = 5e6;
+// The launches the small tiles stand in for: the big tiles (a stage of 256 rows;
+// W16 on 192 columns) and the tile kernel (a 128 x 128 stage and each further
+// 128 x 128 of a larger tile, per turn one workgroup of a CU).
+struct LargeCost { double fixed, stage, end, t_fixed, one, more, t_end, reduce, bytes; };
+constexpr LargeCost kLargeCost[7] = {
+    {3.64, 1.26, 6.72, 3.64, 0.82, 0.37, 3.28, 2.55, 4.14e6},  // G128
+    {5.0, 1.8, 4.0, 0, 0, 0, 0, 0, 1},                         // G64
+    {5.13, 1.0, 7.8, 5.13, 0.61, 0.30, 1.92, 1.72, 2.99e6},    // ROW4
+    {0.0, 1.1, 6.61, 0.0, 0.51, 0.34, 2.51, 7.09, 3.94e6},     // ROW8
+    {5.0, 3.5, 4.0, 0, 0, 0, 0, 0, 1},                         // G32
+    {2.34, 1.49, 7.94, 2.34, 0.64, 0.40, 3.74, 3.28, 4.31e6},  // G128I8
+    {6.81, 1.24, 0.0, 0, 0, 0, 0, 0, 1},                       // W16
+};
 
 bool mid_rounds_ok(int64_t M, int64_t N) {
   return ((M + 255) / 256) * ((N + 191) / 192) <= 2 * (int64_t)ic_num_cus();
@@ -50,16 +72,17 @@ struct MidPlan { int tile, S; double us; };
 MidPlan mid_plan(int mode, int64_t M, int64_t N, int KT, int min_s, int max_s) {
   const int64_t cus = ic_num_cus();
   MidPlan best{0, 1, 1e30};
+  const MidCost& c = kMidCost[mode];
   for (int t = 0; t < kMidTiles; ++t) {
-    const double lat = kMidCost[mode].lat[t], thr = kMidCost[mode].thr[t];
-    if (lat == 0) continue;
+    if (c.lat[t] == 0) continue;
+    const auto stage = [&](int64_t n) { return n * c.thr[t] > c.lat[t] ? n * c.thr[t] : c.lat[t]; };
     const int64_t tiles = ((M + kMidTile[t].bm - 1) / kMidTile[t].bm) * ((N + kMidTile[t].bn - 1) / kMidTile[t].bn);
     for (int S = min_s; S <= max_s && (S == min_s || KT / S >= 4); ++S) {
-      int64_t load = (tiles * S + cus - 1) / cus;
-      if (t == 3 && load > 1) load = (load + 1) & ~1;  // two at a time: an odd one leaves half its CU idle
-      const double per = load * thr > lat ? load * thr : lat;
-      const double us = kMidFixed + (KT + S - 1) / S * per +
-                        (S > 1 ? kMidReduce + (double)S * M * N * 8.0 / kMidBytesPerUs : 0.0);
+      const int64_t load = (tiles * S + cus - 1) / cus, wgs = c.wgs[t] > 0 ? c.wgs[t] : load;
+      const int64_t turns = (load + wgs - 1) / wgs, rest = load % wgs;
+      const double per = (load / wgs) * stage(wgs) + (rest > 0 ? stage(rest) : 0.0);
+      const double us = c.fixed + (KT + S - 1) / S * per + turns * c.end[t] +
+                        (S > 1 ? c.reduce + (double)S * M * N * 8.0 / c.bytes : 0.0);
       if (us < best.us) best = {t, S, us};
     }
   }

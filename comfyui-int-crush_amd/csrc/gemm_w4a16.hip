@@ -389,22 +389,25 @@ hipError_t launch_w16_mid(const u16* A, int64_t lda, const uint8_t* B, int64_t l
   return ic_launch_mid_w16(g, p.tile, p.S, st);
 }
 
-// Small tiles (gemm_mid.h) instead of the 256-row ones, or of the 128 x 256
-// tile for M <= 128, by the estimates of gemm_mid_plan.h: a 256 x 192 tile's
-// 64-K stage takes ~1.2 us, the 128 x 256 tile's ~1.15.
+// Small tiles (gemm_mid.h) instead of the big ones, or of the 128 x 256 tile for
+// M <= 128, by the estimates of gemm_mid_plan.h.  A 64-K stage of the 256-column
+// tiles takes 1.35 of the 192-column ones' (768 x 18432 x 3072: one round of 256
+// x 256, 90 us, where the 192-column estimate of two rounds let 128 x 128 tiles
+// take 140), the three-slot ring's 1.12; the 128 x 256 tile's 1.1 us.
 MidPlan w16_plan(int64_t M, int64_t N, int64_t K, int max_s) {
   MidPlan p = mid_plan(big::W16, M, N, (int)(K / 64), 1, max_s);
+  const LargeCost& c = kLargeCost[big::W16];
   const int64_t cus = ic_num_cus();
-  double base = 1e30;
+  double base;
   if (M > 128) {
-    for (int tmb = 8; tmb <= 10; ++tmb) {
-      const int64_t tiles = ((M + 32 * tmb - 1) / (32 * tmb)) * ((N + big::BN - 1) / big::BN);
-      const double us = (double)((tiles + cus - 1) / cus) * ((double)(K / 64) * 1.2 * tmb / 8.0 + 4.0) + 5.0;
-      if (us < base) base = us;
-    }
+    const W16Big b = w16_big_pick(M, N);
+    const int64_t bm = 32 * b.tmb, bn = b.wide ? 256 : big::BN;
+    const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const double stage = c.stage * b.tmb / 8.0 * (b.wide ? 1.35 : 1.0) * (K > 8192 ? 1.12 : 1.0);
+    base = c.fixed + (double)((tiles + cus - 1) / cus) * ((double)(K / 64) * stage + c.end);
   } else {
     const int64_t tiles = (N + 255) / 256;
-    base = (double)((tiles + cus - 1) / cus) * (double)(K / 64) * 1.15 + 4.0;
+    base = c.fixed + (double)((tiles + cus - 1) / cus) * (double)(K / 64) * 1.1;
   }
   if (base <= p.us || !mid_rounds_ok(M, N)) p.S = 0;  // the other tiles
   return p;

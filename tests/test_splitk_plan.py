@@ -57,3 +57,28 @@ def test_small_tiles_without_a_workspace(rt, weights):
     for M, N, K in ((64, 1024, 1024), (200, 1024, 1024), (256, 4096, 1152)):
         kind, _, _, S = rt.gemm_route(weights, M, N, K, 1, workspace_bytes=0)
         assert (kind, S) == ("small", 1), (M, N, K)
+
+
+@pytest.mark.parametrize("weights,M,N,K,G,us", [
+    # (large, small): measured on MI355X, the launch the small tiles lose to
+    (2, 768, 18432, 3072, 24, (89.8, 140)),    # one round of 256 x 256 tiles
+    (2, 2048, 7688, 2560, 20, (82.3, 121)),
+    (2, 512, 9216, 3072, 24, (64.9, 81)),      # 128 x 64 tiles in two turns per CU
+    (2, 384, 12288, 3072, 24, (64.5, 81)),
+    (2, 1536, 3072, 3072, 24, (63.7, 79.5)),
+    (0, 2048, 12288, 3072, 1, (72.6, 82.2)),
+    (0, 2500, 4096, 1152, 1, (20.5, 23.6)),    # short K: the turns' ends weigh
+    (1, 640, 12288, 3072, 24, (42.9, 48.1)),
+    (1, 384, 18432, 3072, 24, (42.8, 47.6)),
+    (0, 384, 18432, 3072, 24, (43.4, 54.4)),
+])
+def test_large_tiles_kept_where_they_lead(rt, weights, M, N, K, G, us):
+    assert rt.gemm_route(weights, M, N, K, G)[0] in ("big", "tiles"), us
+
+
+@pytest.mark.parametrize("weights,M,N,K,G", [
+    (0, 77, 4096, 4096, 1), (0, 512, 3072, 3072, 1), (1, 64, 9216, 3072, 24), (1, 146, 1312, 8448, 132),
+    (1, 1357, 2560, 7680, 120), (2, 63, 3256, 3712, 29), (2, 292, 2496, 13312, 104), (0, 512, 3072, 3072, 24),
+])
+def test_small_tiles_kept_where_they_lead(rt, weights, M, N, K, G):
+    assert rt.gemm_route(weights, M, N, K, G)[0] == "small"
