@@ -682,42 +682,42 @@ __global__ __launch_bounds__(TH, (RqLds<DT, LOG4R, NT, VAR, TH, NORM>::kMinWaves
     for (int c = 0; c < NT; ++c) {
       if (c * kTile >= K_w) break;  // uniform
       const int o0 = 16 * (t + TH * c);
-      u16 g[16];  // gathered bits (has_perm)
-      v4u ra{}, rb{};
-      if (has_perm) {
-        const char* src = (const char*)rowbuf;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          g[2 * i] = *(const u16*)(src + (po[PLAIN ? 0 : c][i] & 0xffffu));
-          g[2 * i + 1] = *(const u16*)(src + (po[PLAIN ? 0 : c][i] >> 16));
-        }
-      } else if constexpr (WLR) {
-        // this lane's 16 consecutive positions are wave-local 16 lane .. 16 lane + 15
-        const char* wl = slice + wlr_off(c, 16 * lane);
-        ra = *(const v4u*)wl;
-        rb = *(const v4u*)(wl + 16);
-      } else {
-        ra = *(const v4u*)(rowbuf + rbaddr(o0));
-        rb = *(const v4u*)(rowbuf + rbaddr(o0) + 8);
-      }
+      const char* const src = (const char*)rowbuf;
+      const u16* const run = WLR ? (const u16*)(slice + wlr_off(c, 16 * lane))  // wave-local 16 lane .. 16 lane + 15
+                                 : rowbuf + rbaddr(o0);
       if constexpr (QUANT) {
+        // The branches meet in vv alone: the gathered bits kept beside the row's
+        // own until after them were 16 more registers, which the kernels with
+        // either factors or a perm spilled (perm only, bf16: R = 4096, 4096 x
+        // 9216 129 us against 90; R = 1024 with an RMSNorm, 4096 x 6144 102
+        // against 61).
         float vv[16];
         if (has_perm) {
 #pragma unroll
-          for (int j = 0; j < 16; ++j) vv[j] = bits16_f32<DT>(g[j]);
+          for (int i = 0; i < 8; ++i) {
+            vv[2 * i] = bits16_f32<DT>(*(const u16*)(src + (po[PLAIN ? 0 : c][i] & 0xffffu)));
+            vv[2 * i + 1] = bits16_f32<DT>(*(const u16*)(src + (po[PLAIN ? 0 : c][i] >> 16)));
+          }
         } else {
-          unpack8<DT>(ra, vv);
-          unpack8<DT>(rb, vv + 8);
+          unpack8<DT>(*(const v4u*)run, vv);
+          unpack8<DT>(*(const v4u*)(run + 8), vv + 8);
         }
         const v4u codes = quant16(vv, s, rcp_s);
         if (o0 < K_w) *(v4u*)(qrow + o0) = codes;
       } else {
+        v4u ra, rb;
         if (has_perm) {
           uint32_t w[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) w[i] = (uint32_t)g[2 * i] | ((uint32_t)g[2 * i + 1] << 16);
+          for (int i = 0; i < 8; ++i) {
+            const uint32_t lo = *(const u16*)(src + (po[PLAIN ? 0 : c][i] & 0xffffu));
+            w[i] = lo | ((uint32_t)*(const u16*)(src + (po[PLAIN ? 0 : c][i] >> 16)) << 16);
+          }
           ra = v4u{w[0], w[1], w[2], w[3]};
           rb = v4u{w[4], w[5], w[6], w[7]};
+        } else {
+          ra = *(const v4u*)run;
+          rb = *(const v4u*)(run + 8);
         }
         if (o0 < K_w) {
           v4u* dst = (v4u*)(y_out + (int64_t)row * ldy + o0);
