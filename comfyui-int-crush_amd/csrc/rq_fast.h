@@ -152,10 +152,13 @@ struct RqLds {
   // Waves per SIMD that the LDS admits, which the registers then have to (the
   // compiler otherwise took up to 184 and left one workgroup of two or three).
   // At most three (168 registers; four spill), four where two seven-wave
-  // workgroups need them, two for the three tiles of unrotated normalised rows.
+  // workgroups need them, two for the three tiles of unrotated normalised rows,
+  // one for the four tiles of R = 4096 with factors or a perm, whose constants
+  // alone are 96 registers (at two, 75 to 212 spilled: 4096 x 14336, perm only,
+  // f16 151 -> 251 us, bf16 172 -> 289).
   static constexpr int kWgs = occ(XROT ? kXbTight : kXbPad, DBR ? 2 : 1);
   static constexpr int kWaves = (kWgs * (TH / 64) + 3) / 4;
-  static constexpr int kCap = LOG4R == 0 && NORM != 0 && NT == 3 ? 2 : 3;
+  static constexpr int kCap = LOG4R == 6 && NT == 4 && VAR != kRqPlain ? 1 : (LOG4R == 0 && NORM != 0 && NT == 3 ? 2 : 3);
   static constexpr int kMinWaves = kWaves < kCap ? (kWaves < 1 ? 1 : kWaves) : (TH == 448 && NT == 1 && NORM == 0 ? kWaves : kCap);
 };
 

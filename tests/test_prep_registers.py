@@ -1,7 +1,8 @@
 """Registers of the single-pass prep kernels, from the metadata of the code
 objects in the built library: spilled registers are reloaded among the loads of
 the next row, and a row then waits for those.  Kernels with either factors or a
-perm carry no more than their own gather's values.  CPU only."""
+perm carry no more than their own gather's values, and R = 4096 rows of four
+tiles (13312 to 16384 values) have a whole register file per wave.  CPU only."""
 from __future__ import annotations
 
 import re
@@ -80,3 +81,9 @@ def test_three_tiles_across_waves(kernels):
         if key[0] == 1:  # bf16; f16 keeps another part of its constants in scratch
             assert k[".vgpr_spill_count"] <= 35, key
         assert k[".private_segment_fixed_size"] <= 144, key
+
+
+@pytest.mark.parametrize("variant", [GENERAL, BOTH])
+def test_four_tiles_across_waves(kernels, variant):
+    for key, k in _spills(kernels, 6, 4, variant, 256).items():
+        assert k[".private_segment_fixed_size"] == 0, key
