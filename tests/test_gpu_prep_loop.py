@@ -1,0 +1,78 @@
+"""The persistent prep kernels with more rows than resident workgroups, so that
+every workgroup walks several (alternating row buffers, the next row's DMA behind
+this row's stores, no barrier at the top of a row): one to sixteen thousand values,
+with and without quantization, against the one-workgroup-per-row kernel (which an
+unaligned output row stride selects); the normalising kernels against the oracle
+at the first, last and wrapping rows."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DT = {torch.float16: 0, torch.bfloat16: 1}
+
+
+def _rows_for(dev, width):
+    """More than twice the rows that are resident at once: at most 16 waves of
+    1024 values per CU."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    return cus * max(1, 16 // width) * 2 + 77, cus
+
+
+def _x(M, K, dtype, dev, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn(M, K, generator=g, device=dev)
+    x[:, ::61] *= 20.0
+    x *= torch.rand(M, 1, generator=g, device=dev) * 4 + 0.1  # each row its own scale
+    return x.to(dtype)
+
+
+def _prep(rt, K_in, K_w, dtype, dev, use_sr, use_perm):
+    g = torch.Generator(device=dev).manual_seed(K_w)
+    f = torch.exp(torch.randn(K_in, generator=g, device=dev) * 0.5) if use_sr else None
+    p = torch.randperm(K_w, generator=g, device=dev) if use_perm else None
+    return f, p, dict(smoothrot=rt.prepare_factors(f, dtype), perm=rt.prepare_perm(p, K_w))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("R", [0, 16, 64, 256, 1024, 4096])
+@pytest.mark.parametrize("use_sr,use_perm", [(False, False), (True, False), (False, True), (True, True)])
+def test_many_rows_equal_the_general_kernel(rt, dev, dtype, R, use_sr, use_perm):
+    for w in (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16):
+        K_in = 1024 * w - (16 if w % 2 else 0)
+        K_w = -(-K_in // max(R, 16)) * max(R, 16)
+        M, _ = _rows_for(dev, w)
+        x = _x(M, K_in, dtype, dev, w)
+        _, _, kw = _prep(rt, K_in, K_w, dtype, dev, use_sr, use_perm)
+        kw.update(rot_size=R, w_in=K_w)
+        q, s = rt.rotate_quantize(x, **kw)
+        q0, s0 = rt.rotate_quantize(x, x_int8_out=torch.empty(M, K_w + 8, dtype=torch.int8, device=dev)[:, :K_w], **kw)
+        assert torch.equal(s, s0) and torch.equal(q, q0), (w, K_w)
+        y = rt.prepare_activation(x, **kw)
+        y0 = rt.prepare_activation(x, out=torch.empty(M, K_w + 4, dtype=dtype, device=dev)[:, :K_w], **kw)
+        assert torch.equal(y.view(torch.int16), y0.contiguous().view(torch.int16)), (w, K_w)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("norm", ["layer", "rms"])
+@pytest.mark.parametrize("use_sr,use_perm", [(False, False), (True, False), (False, True), (True, True)])
+def test_many_normalised_rows_match_oracle(rt, oracle, dev, dtype, norm, use_sr, use_perm):
+    for R, w in ((16, 1), (256, 2), (64, 3), (0, 4), (256, 5), (1024, 5), (0, 6), (1024, 6), (64, 7), (256, 8), (0, 11),
+                 (256, 12), (1024, 14), (4096, 16)):
+        K_in = 1024 * w - (16 if w % 2 else 0)
+        K_w = -(-K_in // max(R, 16)) * max(R, 16)
+        M, cus = _rows_for(dev, w)
+        x = _x(M, K_in, dtype, dev, w + R)
+        f, p, kw = _prep(rt, K_in, K_w, dtype, dev, use_sr, use_perm)
+        g = torch.Generator(device=dev).manual_seed(1)
+        nw = 1 + 0.2 * torch.randn(K_in, generator=g, device=dev)
+        nb = 0.1 * torch.randn(K_in, generator=g, device=dev)
+        q, s = rt.norm_rotate_quantize(x, norm=norm, weight=nw, bias=nb, eps=1e-6, rot_size=R, w_in=K_w, **kw)
+        rows = sorted({0, M // 2, M - 1} | {cus * n + d for n in (1, 2, 4) for d in (0, 1) if cus * n + d < M})
+        rq, rs = oracle.norm_rotate_quantize(
+            x[rows].cpu(), DT[dtype], norm, nw.cpu().numpy(), nb.cpu().numpy(), 1e-6,
+            smoothrot=f.cpu().numpy() if use_sr else None, rot_size=R, w_in=K_w, perm=p.cpu().numpy() if use_perm else None)
+        assert np.array_equal(s[rows].cpu().numpy(), rs), (R, K_w)
+        assert np.array_equal(q[rows].cpu().numpy(), rq), (R, K_w)
