@@ -191,8 +191,8 @@ struct RqLds {
 // per row and a re-read of factors and perm for each row (rotate_quant_kernel,
 // which still serves the forms this kernel does not take) took 61.9 us for
 // 4608 x 3072 at R = 256 with both, this kernel 27.9 us.
-template <int DT, int LOG4R, int NT, int VAR, int TH, int NORM = 0, bool QUANT = true>
-__global__ __launch_bounds__(TH, (RqLds<DT, LOG4R, NT, VAR, TH, NORM>::kMinWaves)) void rq_fast_kernel(
+template <int DT, int LOG4R, int NT, int VAR, int TH, int NORM, bool QUANT, int WAVES>
+__global__ __launch_bounds__(TH, WAVES) void rq_fast_kernel(
     const u16* __restrict__ x, int64_t ldx, int M, int K_in, int K_r,
     const float* __restrict__ sr_rcp, const float* __restrict__ sr_f, int K_w,
     const int32_t* __restrict__ perm, int8_t* __restrict__ q_out, int64_t ldq,
@@ -830,9 +830,10 @@ int persistent_grid(int threads, int64_t M) {
   return (int)(M < g ? M : g);
 }
 
-template <int DT, int LOG4R, int NT, int VAR, int TH = kThreads, int NORM = 0, bool QUANT = true>
+template <int DT, int LOG4R, int NT, int VAR, int TH, int NORM, bool QUANT,
+          int WAVES = RqLds<DT, LOG4R, NT, VAR, TH, NORM>::kMinWaves>
 hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
-  constexpr auto kern = rq_fast_kernel<DT, LOG4R, NT, VAR, TH, NORM, QUANT>;
+  constexpr auto kern = rq_fast_kernel<DT, LOG4R, NT, VAR, TH, NORM, QUANT, WAVES>;
   const int64_t K_r = LOG4R == 0 ? a.K_in : ((a.K_in + a.rot_size - 1) / a.rot_size) * a.rot_size;
   kern<<<dim3(persistent_grid<kern>(TH, a.M)), dim3(TH), 0, st>>>(
       (const u16*)a.x, a.ldx, (int)a.M, (int)a.K_in, (int)K_r, a.sr_rcp, a.sr_f, (int)a.K_w, a.perm,
@@ -854,9 +855,17 @@ hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
 // bf16 67.8 -> 48.0; R = 1024 with both 87.5 -> 68.5 and 94.0 -> 73.6).  Three
 // tiles of four waves for normalised unrotated rows of nine to twelve thousand
 // values (LayerNorm, 8192 x 10240: 142 -> 123 against twelve waves).
+// R = 1024 behind a norm, rows of five or six thousand values: up to a row per CU
+// one wide tile, since a second tile's exchange only adds to the latency
+// (LayerNorm, bf16 with a perm, 64 rows of 5120: 10.3 -> 7.3 us, of 6144: 10.6 ->
+// 7.4); at six waves, two or four rows per CU, two tiles with the registers of
+// two waves per SIMD (512 rows of 6144 13.2 -> 11.1, 1024 rows 23.2 -> 20.3),
+// where three rows share a CU or many follow those of three waves (without
+// factors, 768 rows 14.4 against 15.7, 4096 rows 55 against 60).
 template <int DT, int LOG4R, int VAR, int NORM = 0, bool QUANT = true>
 hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
 #define IC_RQ(NT, TH) return launch_fast_t<DT, LOG4R, NT, VAR, TH, NORM, QUANT>(a, st)
+  const int64_t cus = ic_num_cus();
   if constexpr (LOG4R <= 5) {
     switch ((a.K_w + 1023) / 1024) {
       case 1: IC_RQ(1, 64);
@@ -865,8 +874,16 @@ hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
       case 4: IC_RQ(1, 256);
       case 5:
         if constexpr (NORM == 0 && LOG4R >= 3) IC_RQ(1, 320);
+        if constexpr (NORM != 0 && LOG4R == 5) {
+          if (a.M <= cus) IC_RQ(1, 320);
+        }
         IC_RQ(2, 192);
       case 6:
+        if constexpr (NORM != 0 && LOG4R == 5) {
+          const int64_t per_cu = (a.M + cus - 1) / cus;
+          if (per_cu <= 1) IC_RQ(1, 384);
+          if (per_cu == 2 || per_cu == 4) return launch_fast_t<DT, LOG4R, 2, VAR, 192, NORM, QUANT, 2>(a, st);
+        }
         if constexpr (NORM == 0 && VAR != kRqPlain && (LOG4R == 3 || LOG4R == 4)) IC_RQ(1, 384);
         IC_RQ(2, 192);
       case 7:

@@ -55,6 +55,33 @@ def test_many_rows_equal_the_general_kernel(rt, dev, dtype, R, use_sr, use_perm)
         assert torch.equal(y.view(torch.int16), y0.contiguous().view(torch.int16)), (w, K_w)
 
 
+def _norm_rows_match(rt, oracle, dev, x, rows, R, K_w, dtype, norm, use_sr, use_perm):
+    K_in = x.shape[1]
+    f, p, kw = _prep(rt, K_in, K_w, dtype, dev, use_sr, use_perm)
+    g = torch.Generator(device=dev).manual_seed(1)
+    nw = 1 + 0.2 * torch.randn(K_in, generator=g, device=dev)
+    nb = 0.1 * torch.randn(K_in, generator=g, device=dev)
+    q, s = rt.norm_rotate_quantize(x, norm=norm, weight=nw, bias=nb, eps=1e-6, rot_size=R, w_in=K_w, **kw)
+    rq, rs = oracle.norm_rotate_quantize(
+        x[rows].cpu(), DT[dtype], norm, nw.cpu().numpy(), nb.cpu().numpy(), 1e-6,
+        smoothrot=f.cpu().numpy() if use_sr else None, rot_size=R, w_in=K_w, perm=p.cpu().numpy() if use_perm else None)
+    assert np.array_equal(s[rows].cpu().numpy(), rs), (R, K_w, x.shape[0])
+    assert np.array_equal(q[rows].cpu().numpy(), rq), (R, K_w, x.shape[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("norm", ["layer", "rms"])
+@pytest.mark.parametrize("use_sr,use_perm", [(False, False), (True, False), (False, True), (True, True)])
+def test_normalised_rows_at_the_width_rules_lines(rt, oracle, dev, dtype, norm, use_sr, use_perm):
+    """R = 1024, five or six thousand values: one wide tile up to a row per CU,
+    two narrow ones beyond, under two register bounds."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    for K_in, K_w in ((4112, 5120), (5120, 5120), (5136, 6144), (6144, 6144)):
+        for M in (1, cus, cus + 1, 2 * cus + 1, 4 * cus, 4 * cus + 1):
+            x = _x(M, K_in, dtype, dev, M)
+            _norm_rows_match(rt, oracle, dev, x, sorted({0, M // 2, M - 1}), 1024, K_w, dtype, norm, use_sr, use_perm)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("norm", ["layer", "rms"])
 @pytest.mark.parametrize("use_sr,use_perm", [(False, False), (True, False), (False, True), (True, True)])
@@ -65,14 +92,5 @@ def test_many_normalised_rows_match_oracle(rt, oracle, dev, dtype, norm, use_sr,
         K_w = -(-K_in // max(R, 16)) * max(R, 16)
         M, cus = _rows_for(dev, w)
         x = _x(M, K_in, dtype, dev, w + R)
-        f, p, kw = _prep(rt, K_in, K_w, dtype, dev, use_sr, use_perm)
-        g = torch.Generator(device=dev).manual_seed(1)
-        nw = 1 + 0.2 * torch.randn(K_in, generator=g, device=dev)
-        nb = 0.1 * torch.randn(K_in, generator=g, device=dev)
-        q, s = rt.norm_rotate_quantize(x, norm=norm, weight=nw, bias=nb, eps=1e-6, rot_size=R, w_in=K_w, **kw)
         rows = sorted({0, M // 2, M - 1} | {cus * n + d for n in (1, 2, 4) for d in (0, 1) if cus * n + d < M})
-        rq, rs = oracle.norm_rotate_quantize(
-            x[rows].cpu(), DT[dtype], norm, nw.cpu().numpy(), nb.cpu().numpy(), 1e-6,
-            smoothrot=f.cpu().numpy() if use_sr else None, rot_size=R, w_in=K_w, perm=p.cpu().numpy() if use_perm else None)
-        assert np.array_equal(s[rows].cpu().numpy(), rs), (R, K_w)
-        assert np.array_equal(q[rows].cpu().numpy(), rq), (R, K_w)
+        _norm_rows_match(rt, oracle, dev, x, rows, R, K_w, dtype, norm, use_sr, use_perm)

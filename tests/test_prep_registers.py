@@ -47,7 +47,7 @@ def _metadata(elf: bytes) -> dict:
 
 @pytest.fixture(scope="module")
 def kernels(rt):
-    """(dtype, log4 R, tiles, variant, threads, norm, quant) -> kernel metadata"""
+    """(dtype, log4 R, tiles, variant, threads, norm, quant, waves) -> kernel metadata"""
     assert rt.KERNELS_AVAILABLE, rt.LOAD_ERROR
     out = {}
     with open(rt.LIB_PATH, "rb") as f:
@@ -56,7 +56,7 @@ def kernels(rt):
         for k in _metadata(elf).get("amdhsa.kernels", []):
             m = _KERNEL.search(k[".name"])
             if m:
-                out[tuple(int(v) for v in re.findall(r"L[ib](\d+)E", m.group(1)))[:7]] = k
+                out[tuple(int(v) for v in re.findall(r"L[ib](\d+)E", m.group(1)))] = k
     assert len(out) > 500
     return out
 
