@@ -152,13 +152,13 @@ struct RqLds {
   // Waves per SIMD that the LDS admits, which the registers then have to (the
   // compiler otherwise took up to 184 and left one workgroup of two or three).
   // At most three (168 registers; four spill), four where two seven-wave
-  // workgroups need them, two for the three tiles of unrotated normalised rows,
+  // workgroups need them, two for the three or four tiles of unrotated rows,
   // one for the four tiles of R = 4096 with factors or a perm, whose constants
   // alone are 96 registers (at two, 75 to 212 spilled: 4096 x 14336, perm only,
   // f16 151 -> 251 us, bf16 172 -> 289).
   static constexpr int kWgs = occ(XROT ? kXbTight : kXbPad, DBR ? 2 : 1);
   static constexpr int kWaves = (kWgs * (TH / 64) + 3) / 4;
-  static constexpr int kCap = LOG4R == 6 && NT == 4 && VAR != kRqPlain ? 1 : (LOG4R == 0 && NORM != 0 && NT == 3 ? 2 : 3);
+  static constexpr int kCap = LOG4R == 6 && NT == 4 && VAR != kRqPlain ? 1 : (LOG4R == 0 && NT >= 3 ? 2 : 3);
   static constexpr int kMinWaves = kWaves < kCap ? (kWaves < 1 ? 1 : kWaves) : (TH == 448 && NT == 1 && NORM == 0 ? kWaves : kCap);
 };
 
@@ -862,9 +862,15 @@ hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
 // two waves per SIMD (512 rows of 6144 13.2 -> 11.1, 1024 rows 23.2 -> 20.3),
 // where three rows share a CU or many follow those of three waves (without
 // factors, 768 rows 14.4 against 15.7, 4096 rows 55 against 60).
+// Unrotated bf16 rows of nine to sixteen thousand values with factors or a perm:
+// three or four tiles of four waves for more than six rows per CU, whose
+// workgroups the wide ones' single one per CU does not overlap (perm only, 4096 x
+// 12288: 40.0 on twelve waves, 36.2 on three tiles, x 16384: 57 and 49; up to
+// there the wide tiles lead, 512 x 12288 9.1 against 10.3.  f16 is level).
 template <int DT, int LOG4R, int VAR, int NORM = 0, bool QUANT = true>
 hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
 #define IC_RQ(NT, TH) return launch_fast_t<DT, LOG4R, NT, VAR, TH, NORM, QUANT>(a, st)
+  constexpr bool kManyUnrotated = LOG4R == 0 && NORM == 0 && QUANT && DT == IC_DTYPE_BF16 && VAR != kRqPlain;
   const int64_t cus = ic_num_cus();
   if constexpr (LOG4R <= 5) {
     switch ((a.K_w + 1023) / 1024) {
@@ -895,11 +901,17 @@ hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
       case 11:
       case 12:
         if constexpr (LOG4R == 0 && NORM != 0) IC_RQ(3, 256);
+        if constexpr (kManyUnrotated) {
+          if (a.M > 6 * cus) IC_RQ(3, 256);
+        }
         IC_RQ(1, 768);
       case 13:
       case 14:
         if constexpr (LOG4R == 5) IC_RQ(2, 448);
         break;
+    }
+    if constexpr (kManyUnrotated) {
+      if (a.M > 6 * cus) IC_RQ(4, 256);
     }
     IC_RQ(2, 512);
   } else {

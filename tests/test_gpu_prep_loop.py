@@ -55,6 +55,21 @@ def test_many_rows_equal_the_general_kernel(rt, dev, dtype, R, use_sr, use_perm)
         assert torch.equal(y.view(torch.int16), y0.contiguous().view(torch.int16)), (w, K_w)
 
 
+@pytest.mark.parametrize("K_in,K_w", [(8208, 8208), (12288, 12288), (12288, 12304), (16384, 16384)])
+@pytest.mark.parametrize("use_sr,use_perm", [(True, False), (False, True), (True, True)])
+def test_unrotated_rows_at_the_width_rules_line(rt, dev, K_in, K_w, use_sr, use_perm):
+    """bf16: wide tiles up to six rows per CU, three or four tiles of four waves
+    beyond."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    for M in (6 * cus, 6 * cus + 1):
+        x = _x(M, K_in, torch.bfloat16, dev, M)
+        _, _, kw = _prep(rt, K_in, K_w, torch.bfloat16, dev, use_sr, use_perm)
+        q, s = rt.rotate_quantize(x, w_in=K_w, **kw)
+        q0, s0 = rt.rotate_quantize(x, w_in=K_w, x_int8_out=torch.empty(M, K_w + 8, dtype=torch.int8, device=dev)[:, :K_w],
+                                    **kw)
+        assert torch.equal(s, s0) and torch.equal(q, q0), M
+
+
 def _norm_rows_match(rt, oracle, dev, x, rows, R, K_w, dtype, norm, use_sr, use_perm):
     K_in = x.shape[1]
     f, p, kw = _prep(rt, K_in, K_w, dtype, dev, use_sr, use_perm)
