@@ -708,19 +708,26 @@ __global__ __launch_bounds__(TH, WAVES) void rq_fast_kernel(
         const v4u codes = quant16(vv, s, rcp_s);
         if (o0 < K_w) *(v4u*)(qrow + o0) = codes;
       } else {
-        v4u ra, rb;
+        // here the pairs are formed after both branches: inside the first one,
+        // unrotated f16 rows with a perm only, 4096 x 16384, took 56 us against 45
+        u16 g[16];
+        v4u ra{}, rb{};
         if (has_perm) {
-          uint32_t w[8];
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            const uint32_t lo = *(const u16*)(src + (po[PLAIN ? 0 : c][i] & 0xffffu));
-            w[i] = lo | ((uint32_t)*(const u16*)(src + (po[PLAIN ? 0 : c][i] >> 16)) << 16);
+            g[2 * i] = *(const u16*)(src + (po[PLAIN ? 0 : c][i] & 0xffffu));
+            g[2 * i + 1] = *(const u16*)(src + (po[PLAIN ? 0 : c][i] >> 16));
           }
-          ra = v4u{w[0], w[1], w[2], w[3]};
-          rb = v4u{w[4], w[5], w[6], w[7]};
         } else {
           ra = *(const v4u*)run;
           rb = *(const v4u*)(run + 8);
+        }
+        if (has_perm) {
+          uint32_t w[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) w[i] = (uint32_t)g[2 * i] | ((uint32_t)g[2 * i + 1] << 16);
+          ra = v4u{w[0], w[1], w[2], w[3]};
+          rb = v4u{w[4], w[5], w[6], w[7]};
         }
         if (o0 < K_w) {
           v4u* dst = (v4u*)(y_out + (int64_t)row * ldy + o0);
