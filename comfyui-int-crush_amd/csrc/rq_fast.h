@@ -680,6 +680,14 @@ __global__ __launch_bounds__(TH, WAVES) void rq_fast_kernel(
     }
 
     // ---- gather + quantize + store 16 codes (or 16 values) per run
+    // kEarlyValues: the gathered bits become values in the perm's branch.  Kept
+    // beside the row's own until after both branches they were 16 more registers,
+    // which the kernels with either factors or a perm spilled (perm only, bf16: R =
+    // 4096, 4096 x 9216 129 us against 90; R = 1024 with an RMSNorm, 4096 x 6144
+    // 102 against 61).  Where those registers are there, after both is the faster
+    // form (perm only, f16: R = 4096, 4096 x 8192 49 against 53 us; not quantized,
+    // unrotated, 4096 x 16384 45 against 56).
+    constexpr bool kEarlyValues = QUANT && (LOG4R <= 5 || NT >= 3);
     int8_t* qrow = q_out + (int64_t)row * ldq;
 #pragma unroll
     for (int c = 0; c < NT; ++c) {
@@ -688,13 +696,8 @@ __global__ __launch_bounds__(TH, WAVES) void rq_fast_kernel(
       const char* const src = (const char*)rowbuf;
       const u16* const run = WLR ? (const u16*)(slice + wlr_off(c, 16 * lane))  // wave-local 16 lane .. 16 lane + 15
                                  : rowbuf + rbaddr(o0);
-      if constexpr (QUANT) {
-        // The branches meet in vv alone: the gathered bits kept beside the row's
-        // own until after them were 16 more registers, which the kernels with
-        // either factors or a perm spilled (perm only, bf16: R = 4096, 4096 x
-        // 9216 129 us against 90; R = 1024 with an RMSNorm, 4096 x 6144 102
-        // against 61).
-        float vv[16];
+      float vv[16];
+      if constexpr (kEarlyValues) {
         if (has_perm) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
@@ -705,11 +708,7 @@ __global__ __launch_bounds__(TH, WAVES) void rq_fast_kernel(
           unpack8<DT>(*(const v4u*)run, vv);
           unpack8<DT>(*(const v4u*)(run + 8), vv + 8);
         }
-        const v4u codes = quant16(vv, s, rcp_s);
-        if (o0 < K_w) *(v4u*)(qrow + o0) = codes;
       } else {
-        // here the pairs are formed after both branches: inside the first one,
-        // unrotated f16 rows with a perm only, 4096 x 16384, took 56 us against 45
         u16 g[16];
         v4u ra{}, rb{};
         if (has_perm) {
@@ -722,18 +721,32 @@ __global__ __launch_bounds__(TH, WAVES) void rq_fast_kernel(
           ra = *(const v4u*)run;
           rb = *(const v4u*)(run + 8);
         }
-        if (has_perm) {
-          uint32_t w[8];
+        if constexpr (QUANT) {
+          if (has_perm) {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) w[i] = (uint32_t)g[2 * i] | ((uint32_t)g[2 * i + 1] << 16);
-          ra = v4u{w[0], w[1], w[2], w[3]};
-          rb = v4u{w[4], w[5], w[6], w[7]};
+            for (int j = 0; j < 16; ++j) vv[j] = bits16_f32<DT>(g[j]);
+          } else {
+            unpack8<DT>(ra, vv);
+            unpack8<DT>(rb, vv + 8);
+          }
+        } else {
+          if (has_perm) {
+            uint32_t w[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) w[i] = (uint32_t)g[2 * i] | ((uint32_t)g[2 * i + 1] << 16);
+            ra = v4u{w[0], w[1], w[2], w[3]};
+            rb = v4u{w[4], w[5], w[6], w[7]};
+          }
+          if (o0 < K_w) {
+            v4u* dst = (v4u*)(y_out + (int64_t)row * ldy + o0);
+            dst[0] = ra;
+            dst[1] = rb;
+          }
         }
-        if (o0 < K_w) {
-          v4u* dst = (v4u*)(y_out + (int64_t)row * ldy + o0);
-          dst[0] = ra;
-          dst[1] = rb;
-        }
+      }
+      if constexpr (QUANT) {
+        const v4u codes = quant16(vv, s, rcp_s);
+        if (o0 < K_w) *(v4u*)(qrow + o0) = codes;
       }
       __builtin_amdgcn_sched_barrier(0);  // one run at a time keeps the register footprint small
     }
