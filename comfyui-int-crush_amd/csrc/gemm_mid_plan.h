@@ -2,9 +2,9 @@
 // shared by the INT8 and W4A16 entry points.
 //
 // Estimated microseconds, fitted to launches timed on MI355X (bf16 outputs, back
-// to back in a graph, weights cycling through three copies; 566 shapes of 17 to
-// 3072 rows, 1024 to 18432 columns and K 1024 to 14336 per mode, each tile and
-// slice count by itself: 5 to 8 % rms).  A CU takes its workgroups in turns of
+// to back in a graph, weights cycling through three copies; 746 shapes of 17 to
+// 3072 rows, 64 to 18432 columns and K 128 to 14336 per mode, each tile and slice
+// count by itself: 5 to 8 % rms).  A CU takes its workgroups in turns of
 // as many as its LDS holds (`wgs`); in a turn of n a stage takes max(lat, n *
 // thr), and a turn ends with `end` (its epilogue).  Where a tile's stage is
 // bound by the VALU's folds (groups of 64 and 32 columns) the turns do not show
@@ -40,13 +40,13 @@ constexpr MidCost kMidCost[7] = {
     {3.0, 2.5, 5.0e6, {0, 0, 0, 0}, {0.39, 0.60, 0.80, 0}, {0.22, 0.33, 0.55, 0}, {0, 0, 0, 0}},  // G64
     {4.50, 2.26, 3.26e6, {5, 3, 2, 0},
      {0.22, 0.28, 0.50, 0}, {0.140, 0.174, 0.358, 0}, {0.36, 0.71, 0.67, 0}},  // ROW4
-    {4.70, 2.94, 4.63e6, {3, 2, 2, 2},
-     {0.19, 0.24, 0.48, 0.77}, {0.167, 0.197, 0.293, 0.423}, {0.10, 0.89, 0.98, 1.51}},  // ROW8
+    {5.57, 3.03, 3.88e6, {3, 2, 2, 2},
+     {0.20, 0.26, 0.45, 0.74}, {0.204, 0.200, 0.309, 0.428}, {0.26, 0.91, 0.86, 1.20}},  // ROW8
     {3.0, 2.5, 5.0e6, {0, 0, 0, 0}, {0.62, 0.95, 1.40, 0}, {0.40, 0.60, 1.05, 0}, {0, 0, 0, 0}},  // G32
     {5.39, 3.41, 5.12e6, {3, 2, 2, 0},
      {0.23, 0.35, 0.54, 0}, {0.193, 0.258, 0.407, 0}, {0.38, 1.36, 1.33, 0}},  // G128I8
-    {6.06, 3.77, 6.49e6, {6, 3, 2, 2},
-     {0.43, 0.44, 0.72, 0.90}, {0.293, 0.300, 0.409, 0.711}, {0, 0, 0.60, 0.13}},  // W16
+    {5.82, 2.96, 5.62e6, {6, 3, 2, 2},
+     {0.43, 0.44, 0.60, 0.90}, {0.294, 0.303, 0.414, 0.711}, {0.02, 0, 0.44, 0.13}},  // W16
 };
 // The launches the small tiles stand in for: the big tiles (a stage of 256 rows;
 // W16 on 192 columns) and the tile kernel (a 128 x 128 stage and each further
@@ -56,10 +56,10 @@ constexpr LargeCost kLargeCost[7] = {
     {3.64, 1.26, 6.72, 3.64, 0.82, 0.37, 3.28, 2.55, 4.14e6},  // G128
     {5.0, 1.8, 4.0, 0, 0, 0, 0, 0, 1},                         // G64
     {5.13, 1.0, 7.8, 5.13, 0.61, 0.30, 1.92, 1.72, 2.99e6},    // ROW4
-    {0.0, 1.1, 6.61, 0.0, 0.51, 0.34, 2.51, 7.09, 3.94e6},     // ROW8
+    {2.17, 1.08, 5.07, 4.88, 0.48, 0.34, 2.19, 6.34, 3.94e6},  // ROW8
     {5.0, 3.5, 4.0, 0, 0, 0, 0, 0, 1},                         // G32
     {2.34, 1.49, 7.94, 2.34, 0.64, 0.40, 3.74, 3.28, 4.31e6},  // G128I8
-    {6.81, 1.24, 0.0, 0, 0, 0, 0, 0, 1},                       // W16
+    {6.92, 1.24, 0.0, 0, 0, 0, 0, 0, 1},                       // W16
 };
 
 bool mid_rounds_ok(int64_t M, int64_t N) {

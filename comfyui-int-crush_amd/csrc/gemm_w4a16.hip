@@ -391,9 +391,9 @@ hipError_t launch_w16_mid(const u16* A, int64_t lda, const uint8_t* B, int64_t l
 
 // Small tiles (gemm_mid.h) instead of the big ones, or of the 128 x 256 tile for
 // M <= 128, by the estimates of gemm_mid_plan.h.  A 64-K stage of the 256-column
-// tiles takes 1.35 of the 192-column ones' (768 x 18432 x 3072: one round of 256
+// tiles takes 1.39 of the 192-column ones' (768 x 18432 x 3072: one round of 256
 // x 256, 90 us, where the 192-column estimate of two rounds let 128 x 128 tiles
-// take 140), the three-slot ring's 1.12; the 128 x 256 tile's 1.1 us.
+// take 140), the three-slot ring's 1.14; the 128 x 256 tile's 1.1 us.
 MidPlan w16_plan(int64_t M, int64_t N, int64_t K, int max_s) {
   MidPlan p = mid_plan(big::W16, M, N, (int)(K / 64), 1, max_s);
   const LargeCost& c = kLargeCost[big::W16];
@@ -403,7 +403,7 @@ MidPlan w16_plan(int64_t M, int64_t N, int64_t K, int max_s) {
     const W16Big b = w16_big_pick(M, N);
     const int64_t bm = 32 * b.tmb, bn = b.wide ? 256 : big::BN;
     const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-    const double stage = c.stage * b.tmb / 8.0 * (b.wide ? 1.35 : 1.0) * (K > 8192 ? 1.12 : 1.0);
+    const double stage = c.stage * b.tmb / 8.0 * (b.wide ? 1.39 : 1.0) * (K > 8192 ? 1.14 : 1.0);
     base = c.fixed + (double)((tiles + cus - 1) / cus) * ((double)(K / 64) * stage + c.end);
   } else {
     const int64_t tiles = (N + 255) / 256;
