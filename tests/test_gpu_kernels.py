@@ -502,8 +502,8 @@ def test_w4a16_dequant_bit_exact_one_hot(rt, oracle, dev, dtype, grouped, M, N):
     """x = one-hot rows (row m selects k = m): each output is a single product
     1 * w[n, m] accumulated in fp32 and rounded to the activation type, so the
     GEMM output equals the kernel's in-LDS dequantized weight, which must be
-    RN_dt(q * RN_dt(s)) bit for bit.  N = 300 takes the direct epilogue, N = 264
-    the LDS-staged one; M = 100 the 128-row tile."""
+    RN_dt(q * RN_dt(s)) bit for bit.  N = 300 takes the 256 x 256 tile and its
+    direct epilogue, N = 264 small tiles."""
     K = 512
     G = K // 128 if grouped else 1
     x = torch.zeros(M, K, dtype=dtype)
@@ -686,7 +686,8 @@ def test_w4a8_big_tile_sampled_rows(rt, oracle, dev, out_dtype, M, N, K, gs):
 
 # 256-, 288- and 320-row tiles (4096, 4608, 5120 rows), ragged in M and N; one
 # and nine 128-K stages (the int8-weight loop alternates two fragment sets by
-# stage and finishes the last stage's deferred block row after the loop)
+# stage and finishes the last stage's deferred block row after the loop; per-row
+# INT4 of one stage takes small tiles)
 ROW_BIG_CASES = [(4096, 3072, 1024), (4608, 3072, 1024), (5120, 3072, 1024), (4600, 3064, 1024),
                  (5100, 3064, 1024), (4608, 3072, 128), (4096, 3072, 1152)]
 
@@ -731,10 +732,10 @@ def test_per_row_big_tile_sampled_rows(rt, oracle, dev, out_dtype, M, N, K, int4
 @pytest.mark.parametrize("M,N,K", [(300, 384, 2048), (64, 3072, 4096), (4608, 3072, 1024), (600, 1000, 1536),
                                    (5, 1000, 1536)])
 def test_w4a8_group_sizes(rt, oracle, dev, gs, M, N, K):
-    """Group sizes other than 128 run the MFMA kernels: multiples of 128
-    (tiled and split-K) fold each 128-column stage, odd multiples of 64 (the
-    288 x 192 kernel's 64-block mode) each 64-K step, odd multiples of 32
-    (its 32-column mode) each 32-column half step, with the scale of the
+    """Group sizes other than 128 run the MFMA kernels, small tiles (some in K
+    slices) and at 4608 rows 288 x 192: multiples of 128 fold each 128-column
+    stage, odd multiples of 64 (the 64-block mode) each 64-K step, odd multiples
+    of 32 (the 32-column mode) each 32-column half step, with the scale of the
     step's group.  Bit-exact against the oracle's epilogue over accumulators
     of gcd(group, 128) columns with the scales repeated."""
     if K % gs:
@@ -803,7 +804,7 @@ def test_w4a8_scalar_kernel_fold_blocks(rt, oracle, dev, gs):
 
 
 @pytest.mark.parametrize("G", [48, 12, 96, 32])  # group sizes 64, 256, 32 and 96 at K = 3072
-@pytest.mark.parametrize("M", [200, 100])  # 256 x 256 and 128 x 256 tiles
+@pytest.mark.parametrize("M", [200, 100])  # groups of 32 and 96: 256 x 256 and 128 x 256 tiles; 64 and 256: small tiles
 def test_w4a16_group_sizes(rt, oracle, dev, G, M):
     N, K = 256, 3072
     x = _acts(M, K, torch.bfloat16, seed=86)
@@ -819,9 +820,9 @@ def test_w4a16_group_sizes(rt, oracle, dev, G, M):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("K,G", [(8192, 64), (8256, 129), (12288, 96)])  # 128, 129 and 192 stages of 64 K
 def test_w4a16_long_k_three_slot_ring(rt, oracle, dev, dtype, K, G):
-    """Long K on the big-tile W4A16 modes: K = 8192 with one DMA stage in
-    flight, K > 8192 with two (per-wave vmcnt counts at each stage top, an odd
-    and an even stage count): within fp32-accumulation tolerance of the
+    """Long K in W4A16, which these few tiles take in K slices on small tiles
+    (an odd and an even stage count; the big tiles' two- and three-slot rings
+    are in test_gpu_gemm_tiles.py): within fp32-accumulation tolerance of the
     dequantized-weight product, and one-hot rows return the dequantized
     weights bit for bit."""
     print(f"[w4a16 long K] K={K} G={G} {dtype}", flush=True)
@@ -845,8 +846,8 @@ def test_w4a16_long_k_three_slot_ring(rt, oracle, dev, dtype, K, G):
 
 @pytest.mark.parametrize("K,G", [(64, 1), (128, 2), (192, 3)])  # one, two and three 64-K stages
 def test_w4a16_big_tiles_short_k(rt, oracle, dev, K, G):
-    """The big-tile W4A16 mode with one to three stages (prologue, first and
-    last stage at once): within fp32-accumulation tolerance of the
+    """W4A16 with one to three stages (prologue, first and last stage at once),
+    on small tiles at this shape: within fp32-accumulation tolerance of the
     dequantized-weight product."""
     M, N = 200, 64
     x = _acts(M, K, torch.float16, seed=140 + K)
@@ -860,16 +861,17 @@ def test_w4a16_big_tiles_short_k(rt, oracle, dev, K, G):
 
 
 @pytest.mark.parametrize("M,N,K,G,dtype,bias", [
-    (300, 200, 512, 4, torch.float16, True),        # ragged M and N, two row tiles
-    (1000, 1048, 1024, 8, torch.bfloat16, False),   # N past a 192-column tile
-    (260, 64, 8256, 129, torch.float16, True),      # K > 8192: the three-slot ring; 64-column groups
-    (4096, 384, 576, 1, torch.bfloat16, True),      # per-row scales, 256-row tiles
+    (300, 200, 512, 4, torch.float16, True),        # ragged M and N
+    (1000, 1048, 1024, 8, torch.bfloat16, False),   # many column tiles, the last ragged
+    (260, 64, 8256, 129, torch.float16, True),      # long K in slices; 64-column groups
+    (4096, 384, 576, 1, torch.bfloat16, True),      # per-row scales, many row tiles
 ])
 def test_w4a16_staged_equals_plain(rt, dev, M, N, K, G, dtype, bias):
     """The staged operand layout (w4a16_stage_layout + gemm_w4a16_staged): the
     copy is the stated permutation of the packed weights and scales, and the
-    GEMM's outputs equal gemm_w4a16's bit for bit (the same big-tile kernel
-    and summation order, other DMA addresses)."""
+    GEMM's outputs equal gemm_w4a16's bit for bit (the same kernel, small tiles
+    at these shapes, and summation order, other DMA addresses; the big tiles are
+    in test_gpu_gemm_tiles.py)."""
     print(f"[w4a16 staged] M={M} N={N} K={K} G={G} {dtype} bias={bias}", flush=True)
     assert rt.w4a16_staged_pays(M, N, K, G)
     x = _acts(M, K, dtype, seed=150).to(dev)

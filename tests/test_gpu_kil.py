@@ -2,10 +2,11 @@
 (ic_int4_interleave_k, ic_gemm_w4a8_kil_ex) and the weights unpacked to int8
 (ic_unpack_int4_to_int8, ic_gemm_w4a8_unpacked_ex).  The repack kernel equals
 the numpy restatement in tests/_w4.py, and W4A8 on either form equals W4A8 on
-the checkpoint order bit for bit on every route -- the 288 x 192 kernel in
-each fold mode, the 256 x 128 / split-K tiles, the GEMV, the scalar kernel --
+the checkpoint order bit for bit on every route -- the small tiles in each fold
+mode and in K slices, the 256 x 128 and 288 x 192 tiles, the GEMV, the scalar kernel --
 with and without the activation / residual epilogue, and through the drop-in
-Linear."""
+Linear.  (The shapes of up to 600 rows take the small tiles; the 288 x 192
+kernel's fold modes on ragged shapes are in test_gpu_gemm_tiles.py.)"""
 from __future__ import annotations
 
 import numpy as np
@@ -44,18 +45,18 @@ def test_interleave_kernel_matches_numpy(rt, dev, N, K):
 
 # (M, N, K, G, out dtype): the route each takes is named after it
 ROUTES = [
-    (600, 384, 1024, 8, torch.bfloat16),    # 288 x 192, fold per 128 columns
-    (600, 384, 1024, 16, torch.float16),    # 288 x 192, fold per 64
-    (600, 384, 1024, 32, torch.bfloat16),   # 288 x 192, fold per 32
-    (600, 384, 1024, 1, torch.bfloat16),    # per-row INT4
+    (600, 384, 1024, 8, torch.bfloat16),    # 32 x 64 tiles, fold per 128 columns
+    (600, 384, 1024, 16, torch.float16),    # 32 x 64 tiles, fold per 64
+    (600, 384, 1024, 32, torch.bfloat16),   # 32 x 64 tiles, fold per 32
+    (600, 384, 1024, 1, torch.bfloat16),    # 32 x 64 tiles, per-row INT4
     (200, 256, 1024, 8, torch.float32),     # 256 x 128 (f32 output)
-    (64, 3072, 3072, 24, torch.bfloat16),   # split-K
+    (64, 3072, 3072, 24, torch.bfloat16),   # small tiles in K slices
     (1, 2304, 3072, 1, torch.bfloat16),     # GEMV
     (5, 512, 1024, 32, torch.float16),      # GEMV, fold per 32
     (16, 256, 3072, 24, torch.float32),     # GEMV, fold per 128
     (37, 96, 520, 1, torch.float16),        # scalar kernel (K not a multiple of 128)
     (37, 96, 520, 65, torch.bfloat16),      # scalar kernel, groups of 8
-    (4608, 3072, 12288, 96, torch.bfloat16),  # C3
+    (4608, 3072, 12288, 96, torch.bfloat16),  # C3: 288 x 192
 ]
 
 
@@ -81,8 +82,8 @@ def test_kil_gemm_equals_plain(rt, dev, M, N, K, G, out_dtype, epi):
 @pytest.mark.parametrize("M,N,K,G,out_dtype", ROUTES)
 @pytest.mark.parametrize("epi", [False, True])
 def test_unpacked_gemm_equals_plain(rt, dev, M, N, K, G, out_dtype, epi):
-    """The unpacked form takes the int8-weight kernels: the 288 x 192 kernel's
-    grouped int8 mode, per-row W8A8, the int8 256 x 128 and split-K tiles, the
+    """The unpacked form takes the int8-weight kernels: the small and 288 x 192
+    tiles' grouped int8 mode, per-row W8A8, the int8 256 x 128 tiles, the
     scalar kernel (the tile kernels also at M <= 16); every one folds in the
     same order as the packed routes."""
     print(f"[unpacked] M={M} N={N} K={K} G={G} out={out_dtype} epi={epi}", flush=True)

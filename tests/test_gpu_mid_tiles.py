@@ -1,5 +1,6 @@
-"""The small-tile GEMM kernel (32..128-row tiles, 17 to a few hundred tokens) at
-the edges of its tiles, rings and K slices.
+"""The small-tile GEMM kernel on 17 to a few hundred tokens: the shapes below
+take its 32 x 64 tile (a few 64 x 64), from one K stage to many and in K slices,
+with groups of one to several stages; test_gpu_gemm_tiles.py has every tile.
 
 INT8 modes: bit-equal to the scalar kernel (unaligned operand rows select it),
 which folds the same blocks in the same order; per-row K splits are exact
