@@ -2,8 +2,8 @@
 // shared by the INT8 and W4A16 entry points.
 //
 // Estimated microseconds, fitted to launches timed on MI355X (bf16 outputs, back
-// to back in a graph, weights cycling through three copies; 746 shapes of 17 to
-// 3072 rows, 64 to 18432 columns and K 128 to 14336 per mode, each tile and slice
+// to back in a graph, weights cycling through three copies; 746 shapes and more of
+// 17 to 3072 rows, 64 to 18432 columns and K 128 to 14336 per mode, each tile and slice
 // count by itself: 5 to 8 % rms).  A CU takes its workgroups in turns of
 // as many as its LDS holds (`wgs`); in a turn of n a stage takes max(lat, n *
 // thr), and a turn ends with `end` (its epilogue).  Where a tile's stage is
@@ -38,8 +38,8 @@ constexpr MidCost kMidCost[7] = {
     {5.66, 2.35, 3.47e6, {4, 3, 2, 0},
      {0.22, 0.42, 0.64, 0}, {0.195, 0.243, 0.405, 0}, {0.27, 0.56, 0.98, 0}},  // G128
     {3.0, 2.5, 5.0e6, {0, 0, 0, 0}, {0.39, 0.60, 0.80, 0}, {0.22, 0.33, 0.55, 0}, {0, 0, 0, 0}},  // G64
-    {4.50, 2.26, 3.26e6, {5, 3, 2, 0},
-     {0.22, 0.28, 0.50, 0}, {0.140, 0.174, 0.358, 0}, {0.36, 0.71, 0.67, 0}},  // ROW4
+    {5.37, 1.87, 3.42e6, {5, 3, 2, 0},
+     {0.21, 0.35, 0.47, 0}, {0.140, 0.186, 0.325, 0}, {0.41, 0.44, 0.54, 0}},  // ROW4
     {5.57, 3.03, 3.88e6, {3, 2, 2, 2},
      {0.20, 0.26, 0.45, 0.74}, {0.204, 0.200, 0.309, 0.428}, {0.26, 0.91, 0.86, 1.20}},  // ROW8
     {3.0, 2.5, 5.0e6, {0, 0, 0, 0}, {0.62, 0.95, 1.40, 0}, {0.40, 0.60, 1.05, 0}, {0, 0, 0, 0}},  // G32
@@ -55,7 +55,7 @@ struct LargeCost { double fixed, stage, end, t_fixed, one, more, t_end, reduce, 
 constexpr LargeCost kLargeCost[7] = {
     {3.64, 1.26, 6.72, 3.64, 0.82, 0.37, 3.28, 2.55, 4.14e6},  // G128
     {5.0, 1.8, 4.0, 0, 0, 0, 0, 0, 1},                         // G64
-    {5.13, 1.0, 7.8, 5.13, 0.61, 0.30, 1.92, 1.72, 2.99e6},    // ROW4
+    {4.90, 0.91, 7.52, 4.88, 0.72, 0.26, 1.84, 1.81, 2.99e6},  // ROW4
     {2.17, 1.08, 5.07, 4.88, 0.48, 0.34, 2.19, 6.34, 3.94e6},  // ROW8
     {5.0, 3.5, 4.0, 0, 0, 0, 0, 0, 1},                         // G32
     {2.34, 1.49, 7.94, 2.34, 0.64, 0.40, 3.74, 3.28, 4.31e6},  // G128I8

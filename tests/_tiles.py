@@ -73,11 +73,17 @@ def big(rt, mode, rows, cols, stages):
     return s and (s[0], s[1], K)
 
 
-def tile_kernel(rt, mode, split):
-    """(M, N, K, slices) of a shape that stays on the tile kernel, in K slices or not."""
+def tile_kernel(rt, mode, split, odd_columns=0):
+    """(M, N, K, slices) of a shape that stays on the tile kernel, in K slices or
+    not; odd_columns: added to a multiple of 8 columns, which no other kernel takes."""
     for K in (3072, 8192, 12288) if split else (384, 1024, 3072):
         for M, N in _candidates(True):
-            route = rt.gemm_route(MODES[mode][0], M, N, K, groups(mode, K))
-            if route[0] == "tiles" and (route[3] > 1) == split and ragged(M, N, route[1], route[2]):
-                return M, N, K, route[3]
+            route = rt.gemm_route(MODES[mode][0], M, N + odd_columns, K, groups(mode, K))
+            if route[0] == "tiles" and (route[3] > 1) == split and ragged(M, N + odd_columns, route[1], route[2]):
+                return M, N + odd_columns, K, route[3]
     return None
+
+
+# per-row INT4 in K slices: the small tiles lead wherever the output is aligned
+TILE_KERNEL = [(mode, split, odd) for mode in ("row8", "row4", "g128", "unpacked") for split in (False, True)
+               for odd in (0, 1, 4) if (mode, split, odd) != ("row4", True, 0)]

@@ -27,10 +27,9 @@ def test_big_tiles_are_reached(rt, mode, rows, cols):
         assert _tiles.big(rt, mode, rows, cols, 129)  # the three-slot ring
 
 
-@pytest.mark.parametrize("mode", ["row8", "row4", "g128", "unpacked"])
-@pytest.mark.parametrize("split", [False, True])
-def test_tile_kernel_is_reached(rt, mode, split):
-    assert _tiles.tile_kernel(rt, mode, split)
+@pytest.mark.parametrize("mode,split,odd", _tiles.TILE_KERNEL)
+def test_tile_kernel_is_reached(rt, mode, split, odd):
+    assert _tiles.tile_kernel(rt, mode, split, odd)
 
 
 def test_other_kernels(rt):

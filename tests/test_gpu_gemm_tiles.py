@@ -125,11 +125,10 @@ def test_big_tile_int8(rt, dev, mode, rows, cols, epi):
     _check_int8(rt, dev, mode, *_tiles.big(rt, mode, rows, cols, 3), epi)
 
 
-@pytest.mark.parametrize("mode", ["row8", "row4", "g128", "unpacked"])
-@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("mode,split,odd", _tiles.TILE_KERNEL)
 @pytest.mark.parametrize("epi", [False, True])
-def test_tile_kernel_int8(rt, dev, mode, split, epi):
-    M, N, K, slices = _tiles.tile_kernel(rt, mode, split)
+def test_tile_kernel_int8(rt, dev, mode, split, odd, epi):
+    M, N, K, slices = _tiles.tile_kernel(rt, mode, split, odd)
     _check_int8(rt, dev, mode, M, N, K, epi, slices)
 
 
