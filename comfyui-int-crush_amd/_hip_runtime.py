@@ -975,12 +975,11 @@ def gemm_w4a16(x: torch.Tensor, w_packed: torch.Tensor, s_w: torch.Tensor,
 
 
 def w4a16_staged_pays(M: int, N: int, K: int, G: int) -> bool:
-    """Whether a W4A16 launch of M x N outputs over K takes the big-tile
-    kernel that reads the staged operand layout (w4a16_stage_layout;
-    ic_gemm_w4a16_staged): M above the GEMV and small-tile range, K and the
-    group size multiples of 64, N a multiple of 8.  There it gives the same
-    outputs bit for bit as gemm_w4a16, in fewer DMA cache-line requests per
-    stage (measured on MI355X: C2 4608 x 12288 x 3072 f16 324 -> 314 us,
+    """Whether a W4A16 launch of M x N outputs over K can read the staged operand
+    layout (w4a16_stage_layout; ic_gemm_w4a16_staged), on big tiles or, where few
+    of them would fill the CUs, small ones: M > 128, K and the group size
+    multiples of 64, N a multiple of 8.  There it gives the same outputs bit for
+    bit as gemm_w4a16, in fewer DMA cache-line requests per stage (measured on MI355X: C2 4608 x 12288 x 3072 f16 324 -> 314 us,
     4096 x 5120 x 5120 bf16 228 -> 211 us)."""
     return M > 128 and K % 64 == 0 and K % G == 0 and (G == 1 or (K // G) % 64 == 0) and N % 8 == 0
 

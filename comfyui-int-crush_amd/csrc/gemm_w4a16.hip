@@ -625,8 +625,8 @@ int ic_gemm_w4a16_staged_ws(const void* x, int dtype, int64_t M, int64_t K, int6
   if (M == 0) return IC_OK;
   if (!x || !w_staged || !s_staged || !out) return ic_set_error(IC_ERR_INVALID_ARG, "%s: null pointer", who);
   const int G = (int)num_groups, gsize = (int)(K / num_groups);
-  // the big tiles' conditions (as in ic_gemm_w4a16), and M above the GEMV
-  // and small-tile range: the staged layout has no other kernel
+  // the big tiles' conditions (as in ic_gemm_w4a16), which the small ones share,
+  // and M above the GEMV's and the 128-row tile's range: neither reads this layout
   const bool ok = M > 128 && K % 64 == 0 && (G == 1 || gsize % 64 == 0) && !((uintptr_t)x & 15) &&
                   !((uintptr_t)w_staged & 15) && !((ldx * 2) & 15) && 320 * ldx * 2 < (1LL << 31) &&
                   N * G < (1LL << 31) && !((uintptr_t)out & 15) && (ldo & 7) == 0 && (N & 7) == 0;

@@ -1,8 +1,9 @@
-// Fast path of the fused prep + quantize (the general kernel and the
+// Fast path of the fused prep, quantized or not (the general kernel and the
 // arithmetic it shares with this one are described in rotate_quant.hip).
 // Included by one translation unit per activation dtype and instantiation set
-// (rq_fast_{f16,bf16}{,_plain,_both}.hip, and rq_norm_{f16,bf16}{,_both}.hip
-// for the normalising variants) so the sets compile in parallel.
+// (rq_fast_{f16,bf16}{,_plain,_both}.hip, rq_norm_{f16,bf16}{,_both}.hip for the
+// normalising variants, and rq_prep_{f16,bf16}{,_both}.hip for those that leave
+// the prepared row unquantized) so the sets compile in parallel.
 #pragma once
 #include "rq_common.h"
 
@@ -11,7 +12,8 @@ using namespace rq;
 
 // ===================================================================== fast path
 // 16-bit activations with K_in % 16 == 0, K_w % 16 == 0, 16-byte aligned rows,
-// factor and perm arrays, quantized output, no old-SmoothQuant divide.  Same
+// factor and perm arrays, no old-SmoothQuant divide; the output is quantized, or
+// (QUANT false) the prepared row in the activation type.  Same
 // arithmetic as rotate_quant_kernel, arranged for throughput:
 //   * persistent workgroups walk rows r = blockIdx.x, +gridDim.x, ...; the
 //     SmoothRot reciprocals of a thread's input positions and the gather
