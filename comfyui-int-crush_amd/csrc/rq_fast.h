@@ -884,6 +884,9 @@ hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
 // two waves per SIMD (512 rows of 6144 13.2 -> 11.1, 1024 rows 23.2 -> 20.3),
 // where three rows share a CU or many follow those of three waves (without
 // factors, 768 rows 14.4 against 15.7, 4096 rows 55 against 60).
+// R = 4096 behind a norm, one tile: the registers of two waves per SIMD for up to
+// two rows per CU, which they hold at once, and for four (LayerNorm, bf16, 512 x
+// 4096: 8.7 -> 7.8 us; 4096 rows take 44 on them and 40.5 on three).
 // Unrotated bf16 rows of nine to sixteen thousand values with factors or a perm:
 // three or four tiles of four waves for more than six rows per CU, whose
 // workgroups the wide ones' single one per CU does not overlap (perm only, 4096 x
@@ -937,6 +940,11 @@ hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
     }
     IC_RQ(2, 512);
   } else {
+    if constexpr (NORM != 0) {
+      const int64_t per_cu = (a.M + cus - 1) / cus;
+      if (a.K_w <= kTile && (per_cu <= 2 || per_cu == 4))
+        return launch_fast_t<DT, LOG4R, 1, VAR, kThreads, NORM, QUANT, 2>(a, st);
+    }
     if (a.K_w <= kTile) IC_RQ(1, kThreads);
     if (a.K_w <= 2 * kTile) IC_RQ(2, kThreads);
     if (a.K_w <= 3 * kTile) IC_RQ(3, kThreads);

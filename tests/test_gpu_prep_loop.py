@@ -89,12 +89,17 @@ def _norm_rows_match(rt, oracle, dev, x, rows, R, K_w, dtype, norm, use_sr, use_
 @pytest.mark.parametrize("use_sr,use_perm", [(False, False), (True, False), (False, True), (True, True)])
 def test_normalised_rows_at_the_width_rules_lines(rt, oracle, dev, dtype, norm, use_sr, use_perm):
     """R = 1024, five or six thousand values: one wide tile up to a row per CU,
-    two narrow ones beyond, under two register bounds."""
+    two narrow ones beyond, under two register bounds; R = 4096, one tile: two
+    bounds as well."""
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     for K_in, K_w in ((4112, 5120), (5120, 5120), (5136, 6144), (6144, 6144)):
         for M in (1, cus, cus + 1, 2 * cus + 1, 4 * cus, 4 * cus + 1):
             x = _x(M, K_in, dtype, dev, M)
             _norm_rows_match(rt, oracle, dev, x, sorted({0, M // 2, M - 1}), 1024, K_w, dtype, norm, use_sr, use_perm)
+    for K_in in (1040, 4096):
+        for M in (1, 2 * cus, 2 * cus + 1, 4 * cus, 4 * cus + 1):
+            x = _x(M, K_in, dtype, dev, M)
+            _norm_rows_match(rt, oracle, dev, x, sorted({0, M // 2, M - 1}), 4096, 4096, dtype, norm, use_sr, use_perm)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
