@@ -153,11 +153,13 @@ struct RqLds {
   static constexpr bool DBR = LOG4R <= 5 && (WLR || dbr_fits(XROT ? kXbTight : kXbPad));
   // Waves per SIMD that the LDS admits, which the registers then have to (the
   // compiler otherwise took up to 184 and left one workgroup of two or three).
-  // At most three (168 registers; four spill), four where two seven-wave
-  // workgroups need them, two for the three or four tiles of unrotated rows,
-  // one for the four tiles of R = 4096 with factors or a perm, whose constants
-  // alone are 96 registers (at two, 75 to 212 spilled: 4096 x 14336, perm only,
-  // f16 151 -> 251 us, bf16 172 -> 289).
+  // At most three (168 registers, of which the two narrow tiles behind a norm and
+  // those of R = 1024 spill up to 24 and still lead for many rows, see
+  // launch_fast_nt; four spill more), four where two seven-wave workgroups need
+  // them, two for the three or four tiles of unrotated rows, one for the four
+  // tiles of R = 4096 with factors or a perm, whose constants alone are 96
+  // registers (at two, 75 to 212 spilled: 4096 x 14336, perm only, f16 151 -> 251
+  // us, bf16 172 -> 289).
   static constexpr int kWgs = occ(XROT ? kXbTight : kXbPad, DBR ? 2 : 1);
   static constexpr int kWaves = (kWgs * (TH / 64) + 3) / 4;
   static constexpr int kCap = LOG4R == 6 && NT == 4 && VAR != kRqPlain ? 1 : (LOG4R == 0 && NT >= 3 ? 2 : 3);
@@ -688,8 +690,15 @@ __global__ __launch_bounds__(TH, WAVES) void rq_fast_kernel(
     // 4096, 4096 x 9216 129 us against 90; R = 1024 with an RMSNorm, 4096 x 6144
     // 102 against 61).  Where those registers are there, after both is the faster
     // form (perm only, f16: R = 4096, 4096 x 8192 49 against 53 us; not quantized,
-    // unrotated, 4096 x 16384 45 against 56).
-    constexpr bool kEarlyValues = QUANT && (LOG4R <= 5 || NT >= 3);
+    // unrotated, 4096 x 16384 45 against 56).  So it is on one narrow tile, whose
+    // registers then keep a SIMD at three waves: at four each row is slower (R =
+    // 1024, perm only, bf16 16384 x 1024 30 against 23.4 us, f16 behind a LayerNorm
+    // 36.8 against 28.1), except bf16 behind a norm at R = 64 and 256, where it
+    // spilled; as R = 4096 does there on one tile (RMSNorm, bf16 with a perm, 4608 x
+    // 2048).
+    constexpr bool kOneNarrowTile = NT == 1 && TH <= 256 &&
+                                    !(DT == IC_DTYPE_BF16 && NORM != 0 && (LOG4R == 3 || LOG4R == 4) && !XROT);
+    constexpr bool kEarlyValues = QUANT && (LOG4R <= 5 ? !kOneNarrowTile : NT >= 3 || (NT == 1 && NORM != 0));
     int8_t* qrow = q_out + (int64_t)row * ldq;
 #pragma unroll
     for (int c = 0; c < NT; ++c) {

@@ -87,3 +87,18 @@ def test_three_tiles_across_waves(kernels):
 def test_four_tiles_across_waves(kernels, variant):
     for key, k in _spills(kernels, 6, 4, variant, 256).items():
         assert k[".private_segment_fixed_size"] == 0, key
+
+
+@pytest.mark.parametrize("threads", [64, 128, 256])
+def test_one_narrow_tile_keeps_three_waves(kernels, threads):
+    """R = 1024 with factors or a perm: bf16, and f16 behind a norm, hold more than
+    128 registers (three waves per SIMD), which many short rows run faster on."""
+    for key, k in _spills(kernels, 5, 1, GENERAL, threads).items():
+        if key[6] and (key[0] == 1 or key[5]):
+            assert k[".vgpr_count"] > 128 and k[".vgpr_spill_count"] == 0, key
+
+
+def test_one_tile_across_waves_behind_a_norm(kernels):
+    for key, k in _spills(kernels, 6, 1, GENERAL, 256).items():
+        if key[5]:
+            assert k[".vgpr_spill_count"] == 0, key
