@@ -886,6 +886,10 @@ hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
 // bf16 67.8 -> 48.0; R = 1024 with both 87.5 -> 68.5 and 94.0 -> 73.6).  Three
 // tiles of four waves for normalised unrotated rows of nine to twelve thousand
 // values (LayerNorm, 8192 x 10240: 142 -> 123 against twelve waves).
+// R = 64 and 256, rows of five thousand values: one wide tile up to three rows per
+// CU (R = 256, bf16 without factors and perm, 512 x 5120: 6.2 against 7.4 us), two
+// narrow ones beyond, of which more workgroups share a CU (768 rows level, 1024:
+// 10.9 -> 9.5, 4096: 32.9 -> 27.6; f16 29.6 -> 25.0; f16 with factors or a perm is level).
 // R = 1024 behind a norm, rows of five or six thousand values: up to a row per CU
 // one wide tile, since a second tile's exchange only adds to the latency
 // (LayerNorm, bf16 with a perm, 64 rows of 5120: 10.3 -> 7.3 us, of 6144: 10.6 ->
@@ -913,6 +917,9 @@ hipError_t launch_fast_nt(const ic_rotq_args& a, hipStream_t st) {
       case 3: IC_RQ(1, 192);
       case 4: IC_RQ(1, 256);
       case 5:
+        if constexpr (NORM == 0 && QUANT && (LOG4R == 3 || LOG4R == 4) && (VAR == kRqPlain || DT == IC_DTYPE_BF16)) {
+          if (a.M > 3 * cus) IC_RQ(2, 192);
+        }
         if constexpr (NORM == 0 && LOG4R >= 3) IC_RQ(1, 320);
         if constexpr (NORM != 0 && LOG4R == 5) {
           if (a.M <= cus) IC_RQ(1, 320);

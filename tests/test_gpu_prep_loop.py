@@ -70,6 +70,23 @@ def test_unrotated_rows_at_the_width_rules_line(rt, dev, K_in, K_w, use_sr, use_
         assert torch.equal(s, s0) and torch.equal(q, q0), M
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("R", [64, 256])
+@pytest.mark.parametrize("use_sr,use_perm", [(False, False), (True, False), (False, True), (True, True)])
+def test_five_thousand_values_at_the_width_rules_line(rt, dev, dtype, R, use_sr, use_perm):
+    """One wide tile up to three rows per CU, two narrow ones beyond."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    for K_in in (4112, 5120):
+        K_w = -(-K_in // R) * R
+        for M in (3 * cus, 3 * cus + 1, 7 * cus + 1):
+            x = _x(M, K_in, dtype, dev, M)
+            _, _, kw = _prep(rt, K_in, K_w, dtype, dev, use_sr, use_perm)
+            q, s = rt.rotate_quantize(x, rot_size=R, w_in=K_w, **kw)
+            q0, s0 = rt.rotate_quantize(x, rot_size=R, w_in=K_w,
+                                        x_int8_out=torch.empty(M, K_w + 8, dtype=torch.int8, device=dev)[:, :K_w], **kw)
+            assert torch.equal(s, s0) and torch.equal(q, q0), (M, K_in)
+
+
 def _norm_rows_match(rt, oracle, dev, x, rows, R, K_w, dtype, norm, use_sr, use_perm):
     K_in = x.shape[1]
     f, p, kw = _prep(rt, K_in, K_w, dtype, dev, use_sr, use_perm)
