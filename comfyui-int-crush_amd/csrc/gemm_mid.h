@@ -378,7 +378,7 @@ template <int T, int MODE, int OUT_DT, bool EPI, bool KIL, bool PART>
 hipError_t launch_mid_k(const ic_gemm::GemmArgs& g, int S, hipStream_t st) {
   using CF = MidCfg<T, MODE>;
   // LDS goes in 512-byte granules; the registers (at most 116) hold as many workgroups
-  static_assert(kMidCost[MODE].wgs[T] == 0 || kMidCost[MODE].wgs[T] == 163840 / ((CF::lds_bytes + 511) / 512 * 512),
+  static_assert(kMidCost[MODE].wgs[T] == 163840 / ((CF::lds_bytes + 511) / 512 * 512),
                 "the plan's workgroups per CU");
   const int tiles = ((g.M + CF::BM - 1) / CF::BM) * ((g.N + CF::BN - 1) / CF::BN);
   auto kern = gemm_mid_kernel<CF, OUT_DT, EPI, KIL, PART>;
@@ -415,7 +415,9 @@ hipError_t launch_mid_d(const ic_gemm::GemmArgs& g, int tile, int S, hipStream_t
   switch (tile) {
     case 0: return launch_mid_t<0, MODE, KIL, OUT_DT>(g, S, st);
     case 1: return launch_mid_t<1, MODE, KIL, OUT_DT>(g, S, st);
-    case 2: return launch_mid_t<2, MODE, KIL, OUT_DT>(g, S, st);
+    case 2:
+      if constexpr (MODE != big::ROW4) return launch_mid_t<2, MODE, KIL, OUT_DT>(g, S, st);
+      break;
     case 3:
       if constexpr (MODE == big::ROW8 || MODE == big::W16) return launch_mid_t<3, MODE, KIL, OUT_DT>(g, S, st);
   }

@@ -1,17 +1,20 @@
 // Choice of the small-tile kernel (gemm_mid.h) and its K split: host logic
 // shared by the INT8 and W4A16 entry points.
 //
-// Estimated microseconds, fitted to launches timed on MI355X (bf16 outputs, back
-// to back in a graph, weights cycling through three copies; 746 shapes and more of
-// 17 to 3072 rows, 64 to 18432 columns and K 128 to 14336 per mode, each tile and slice
-// count by itself: 5 to 8 % rms).  A CU takes its workgroups in turns of
+// Estimated microseconds, their constants set so that the choice they lead to is
+// right on launches timed on MI355X (bf16 outputs, back to back in a graph, weights
+// cycling through three copies; 1700 shapes per mode, W4A16 746, of 17 to 4608
+// rows, 64 to 18432 columns and K 128 to 14336, each tile by itself: of 11914
+// launches 12 were more than 4 % slower than the large tiles, by at most 9 %, and 59
+// more than 6 % slower than the best tile).  A CU takes its workgroups in turns of
 // as many as its LDS holds (`wgs`); in a turn of n a stage takes max(lat, n *
-// thr), and a turn ends with `end` (its epilogue).  Where a tile's stage is
-// bound by the VALU's folds (groups of 64 and 32 columns) the turns do not show
-// and wgs is 0, any number at once.
+// thr), and a turn ends with `end` (its epilogue).
 //   W4A16  512 x 9216 x 3072: 128 x 64 tiles, three per CU in two turns, 81 us;
 //          256 x 192 tiles 65 (128 x 128: 71)
 //   W4A16  768 x 18432 x 3072: 128 x 128 139; 256 x 256 tiles in one turn 90
+//   per-row INT4, 4608 x 5120 x 512: 128 x 64 tiles in six turns, whose ends weigh
+//          at short K, 34.6; 256 x 192 25.1
+//   g64    513 x 18432 x 512: 128 x 64 24; 256 x 192 18.1
 //   W8A8   2048 x 12288 x 3072: 128 x 128 82; 256 x 192 72.6; 512 x 3072 x 3072:
 //          64 x 64 tiles 12.8, 256 x 192 in two slices 25.4
 //   g128   640 x 12288 x 3072: 128 x 64 48; 256 x 192 43
@@ -30,21 +33,23 @@ constexpr MidTile kMidTile[kMidTiles] = {{32, 64}, {64, 64}, {128, 64}, {128, 12
 
 struct MidCost {
   double fixed, reduce, bytes;  // of a launch; a split's second kernel, and its partials (8 bytes each) per us
-  int wgs[kMidTiles];
+  int wgs[kMidTiles];  // workgroups that a CU's LDS holds
   double lat[kMidTiles], thr[kMidTiles], end[kMidTiles];  // lat 0: the mode has no such tile
 };
 // by weight mode (big::G128 ... big::W16): 128-K stages, 64-K for W16
 constexpr MidCost kMidCost[7] = {
-    {5.66, 2.35, 3.47e6, {4, 3, 2, 0},
-     {0.22, 0.42, 0.64, 0}, {0.195, 0.243, 0.405, 0}, {0.27, 0.56, 0.98, 0}},  // G128
-    {3.0, 2.5, 5.0e6, {0, 0, 0, 0}, {0.39, 0.60, 0.80, 0}, {0.22, 0.33, 0.55, 0}, {0, 0, 0, 0}},  // G64
-    {5.37, 1.87, 3.42e6, {5, 3, 2, 0},
-     {0.21, 0.35, 0.47, 0}, {0.140, 0.186, 0.325, 0}, {0.41, 0.44, 0.54, 0}},  // ROW4
-    {5.57, 3.03, 3.88e6, {3, 2, 2, 2},
-     {0.20, 0.26, 0.45, 0.74}, {0.204, 0.200, 0.309, 0.428}, {0.26, 0.91, 0.86, 1.20}},  // ROW8
-    {3.0, 2.5, 5.0e6, {0, 0, 0, 0}, {0.62, 0.95, 1.40, 0}, {0.40, 0.60, 1.05, 0}, {0, 0, 0, 0}},  // G32
-    {5.39, 3.41, 5.12e6, {3, 2, 2, 0},
-     {0.23, 0.35, 0.54, 0}, {0.193, 0.258, 0.407, 0}, {0.38, 1.36, 1.33, 0}},  // G128I8
+    {3.45, 2.81, 3.63e6, {4, 3, 2, 0},
+     {0.219, 0.407, 0.728, 0}, {0.205, 0.272, 0.41, 0}, {0.873, 0.973, 1.813, 0}},  // G128
+    {1.98, 5.69, 11.45e6, {4, 3, 2, 0},
+     {0.506, 0.58, 0.82, 0}, {0.241, 0.361, 0.642, 0}, {1.729, 1.736, 1.797, 0}},  // G64
+    {6.12, 1.87, 3.42e6, {5, 3, 0, 0},
+     {0.21, 0.35, 0, 0}, {0.140, 0.186, 0, 0}, {0.605, 0.61, 0, 0}},  // ROW4 (128 x 64 led at 8 of 1718 shapes, by 3 to 5 %: left out)
+    {4.88, 3.03, 3.88e6, {3, 2, 2, 2},
+     {0.20, 0.26, 0.45, 0.74}, {0.204, 0.200, 0.309, 0.428}, {0.279, 1.206, 1.694, 2.295}},  // ROW8
+    {3.05, 1.65, 3.39e6, {4, 3, 2, 0},
+     {0.704, 0.702, 1.298, 0}, {0.349, 0.557, 1.183, 0}, {1.458, 1.72, 2.974, 0}},  // G32
+    {4.73, 3.64, 6.08e6, {3, 2, 2, 0},
+     {0.299, 0.548, 0.599, 0}, {0.193, 0.268, 0.382, 0}, {0.516, 1.208, 1.409, 0}},  // G128I8
     {5.82, 2.96, 5.62e6, {6, 3, 2, 2},
      {0.43, 0.44, 0.60, 0.90}, {0.294, 0.303, 0.414, 0.711}, {0.02, 0, 0.44, 0.13}},  // W16
 };
@@ -53,13 +58,13 @@ constexpr MidCost kMidCost[7] = {
 // 128 x 128 of a larger tile, per turn one workgroup of a CU).
 struct LargeCost { double fixed, stage, end, t_fixed, one, more, t_end, reduce, bytes; };
 constexpr LargeCost kLargeCost[7] = {
-    {3.64, 1.26, 6.72, 3.64, 0.82, 0.37, 3.28, 2.55, 4.14e6},  // G128
-    {5.0, 1.8, 4.0, 0, 0, 0, 0, 0, 1},                         // G64
-    {4.90, 0.91, 7.52, 4.88, 0.72, 0.26, 1.84, 1.81, 2.99e6},  // ROW4
-    {2.17, 1.08, 5.07, 4.88, 0.48, 0.34, 2.19, 6.34, 3.94e6},  // ROW8
-    {5.0, 3.5, 4.0, 0, 0, 0, 0, 0, 1},                         // G32
-    {2.34, 1.49, 7.94, 2.34, 0.64, 0.40, 3.74, 3.28, 4.31e6},  // G128I8
-    {6.92, 1.24, 0.0, 0, 0, 0, 0, 0, 1},                       // W16
+    {1.821, 1.651, 4.001, 2.496, 0.843, 0.396, 3.354, 4.245, 4.762e6},  // G128
+    {0.18, 2.34, 4.939, 0, 0, 0, 0, 0, 1},  // G64
+    {2.19, 1.198, 5.191, 6.188, 0.695, 0.216, 1.296, 3.453, 4.185e6},  // ROW4
+    {4.005, 1.094, 4.838, 4.318, 0.382, 0.394, 2.022, 5.927, 4.962e6},  // ROW8
+    {0.136, 4.487, 7.407, 0, 0, 0, 0, 0, 1},  // G32
+    {3.027, 1.518, 4.94, 2.34, 0.546, 0.533, 3.74, 3.28, 4.965e6},  // G128I8
+    {6.92, 1.24, 0.0, 0, 0, 0, 0, 0, 1},  // W16
 };
 
 bool mid_rounds_ok(int64_t M, int64_t N) {
@@ -78,7 +83,7 @@ MidPlan mid_plan(int mode, int64_t M, int64_t N, int KT, int min_s, int max_s) {
     const auto stage = [&](int64_t n) { return n * c.thr[t] > c.lat[t] ? n * c.thr[t] : c.lat[t]; };
     const int64_t tiles = ((M + kMidTile[t].bm - 1) / kMidTile[t].bm) * ((N + kMidTile[t].bn - 1) / kMidTile[t].bn);
     for (int S = min_s; S <= max_s && (S == min_s || KT / S >= 4); ++S) {
-      const int64_t load = (tiles * S + cus - 1) / cus, wgs = c.wgs[t] > 0 ? c.wgs[t] : load;
+      const int64_t load = (tiles * S + cus - 1) / cus, wgs = c.wgs[t];
       const int64_t turns = (load + wgs - 1) / wgs, rest = load % wgs;
       const double per = (load / wgs) * stage(wgs) + (rest > 0 ? stage(rest) : 0.0);
       const double us = c.fixed + (KT + S - 1) / S * per + turns * c.end[t] +

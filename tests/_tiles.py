@@ -45,7 +45,7 @@ def find(rt, mode: str, kind: str, rows: int, cols: int, K: int, split: bool | N
 
 # tiles each mode has
 SMALL_TILES = [(mode, *tile) for mode in MODES for tile in ((32, 64), (64, 64), (128, 64), (128, 128))
-               if tile != (128, 128) or mode in ("row8", "w4a16")]
+               if tile[0] < 128 or mode in ("row8", "w4a16") or (tile == (128, 64) and mode != "row4")]
 # a mode's tiles that K is split on by the plan of some candidate
 SPLIT_TILES = [("row8", 32, 64), ("row8", 64, 64), ("row8", 128, 64), ("row8", 128, 128), ("row4", 32, 64), ("row4", 64, 64),
                ("g128", 32, 64), ("g128", 64, 64), ("g128", 128, 64), ("unpacked", 32, 64), ("unpacked", 64, 64),
@@ -84,6 +84,6 @@ def tile_kernel(rt, mode, split, odd_columns=0):
     return None
 
 
-# per-row INT4 in K slices: the small tiles lead wherever the output is aligned
+# packed INT4 in K slices: the small tiles lead wherever the output is aligned
 TILE_KERNEL = [(mode, split, odd) for mode in ("row8", "row4", "g128", "unpacked") for split in (False, True)
-               for odd in (0, 1, 4) if (mode, split, odd) != ("row4", True, 0)]
+               for odd in (0, 1, 4) if (mode, split, odd) not in (("row4", True, 0), ("g128", True, 0))]

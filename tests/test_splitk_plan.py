@@ -70,10 +70,21 @@ def test_small_tiles_without_a_workspace(rt, weights):
     (0, 2500, 4096, 1152, 1, (20.5, 23.6)),    # short K: the turns' ends weigh
     (1, 640, 12288, 3072, 24, (42.9, 48.1)),
     (1, 384, 18432, 3072, 24, (42.8, 47.6)),
-    (0, 384, 18432, 3072, 24, (43.4, 54.4)),
+    (1, 4608, 5120, 512, 1, (25.1, 34.6)),     # turns of few stages: their ends weigh
+    (1, 1845, 12288, 512, 1, (27.6, 37.9)),
+    (1, 4096, 5120, 1024, 1, (33.3, 43.4)),
+    (1, 513, 18432, 512, 8, (18.1, 24.0)),     # groups of 64
+    (1, 3072, 3904, 256, 8, (18.8, 25.1)),     # groups of 32
+    (1, 4608, 5120, 256, 2, (23.5, 29.8)),
 ])
 def test_large_tiles_kept_where_they_lead(rt, weights, M, N, K, G, us):
     assert rt.gemm_route(weights, M, N, K, G)[0] in ("big", "tiles"), us
+
+
+def test_unpacked_groups_not_on_the_slower_small_tile(rt):
+    """384 x 18432 x 3072, int8 weights in groups: 64 x 64 tiles 57 us, 128 x 64
+    45.6 and 256 x 192 46.8, which are level."""
+    assert rt.gemm_route(0, 384, 18432, 3072, 24)[1:3] in ((128, 64), (256, 192))
 
 
 @pytest.mark.parametrize("weights,M,N,K,G", [
