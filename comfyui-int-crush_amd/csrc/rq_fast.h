@@ -889,7 +889,9 @@ hipError_t launch_fast_t(const ic_rotq_args& a, hipStream_t st) {
 // R = 64 and 256, rows of five thousand values: one wide tile up to three rows per
 // CU (R = 256, bf16 without factors and perm, 512 x 5120: 6.2 against 7.4 us), two
 // narrow ones beyond, of which more workgroups share a CU (768 rows level, 1024:
-// 10.9 -> 9.5, 4096: 32.9 -> 27.6; f16 29.6 -> 25.0; f16 with factors or a perm is level).
+// 10.9 -> 9.5, 4096: 32.9 -> 27.6, with factors and perm 42.0 -> 32.6; f16 without
+// them 29.6 -> 25.0).  f16 with factors or a perm keeps the wide one: two narrow
+// ones are not measured there.
 // R = 1024 behind a norm, rows of five or six thousand values: up to a row per CU
 // one wide tile, since a second tile's exchange only adds to the latency
 // (LayerNorm, bf16 with a perm, 64 rows of 5120: 10.3 -> 7.3 us, of 6144: 10.6 ->
